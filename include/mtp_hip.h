@@ -425,13 +425,23 @@ int mtp_fused_causal_attention(const void *q, int dtype, int64_t B, int64_t H,
  * Replaces fused_causal_attention_fp8(q, k_fp8, v_fp8, kscale, vscale,
  * scale=None) (mtp_kernels.py:1105-1133; kernel 373-427; eager 817-829):
  * k / v fp8 e4m3fn [B, H, L, D] dequantised per head by kscale[H] /
- * vscale[H] (fp32); q / out [B, H, D] in dtype. No workspace.
+ * vscale[H] (fp32); q / out [B, H, D] in dtype. No workspace: the keys of a
+ * (batch, head) are read by one workgroup.
  */
 int mtp_fused_causal_attention_fp8(const void *q, int dtype, int64_t B,
                                    int64_t H, int64_t D, const void *k_fp8,
                                    const void *v_fp8, int64_t L,
                                    const float *kscale, const float *vscale,
                                    float scale, void *out, void *stream);
+/* The same with a workspace (mtp_attention_workspace_bytes(dtype, B, 1, H, D,
+ * 0, L)): few (batch, head) pairs then spread their keys over the chip. A
+ * missing or smaller workspace is no error (the call runs as the one above). */
+int mtp_fused_causal_attention_fp8_ws(const void *q, int dtype, int64_t B,
+                                      int64_t H, int64_t D, const void *k_fp8,
+                                      const void *v_fp8, int64_t L,
+                                      const float *kscale, const float *vscale,
+                                      float scale, void *out, void *workspace,
+                                      size_t workspace_bytes, void *stream);
 
 /*
  * Replaces fused_tree_attn_rmsnorm_linear(q, k, v, mask, proj_w, rms_w=None,

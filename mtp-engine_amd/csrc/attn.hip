@@ -1,6 +1,7 @@
 // Instantiations of the attention kernels (attn.hpp).
 #include "attn.hpp"
 #include "attn2.hpp"
+#include "attn_dec.hpp"
 
 namespace mtp {
 
@@ -35,6 +36,27 @@ AttnKernel attn2_pick(int ct) {
   return nullptr;
 }
 int attn2_lds_bytes() { return kAttn2Lds; }
+
+namespace {
+template <int KT, bool CTX>
+void (*dec_pick(int d))(AttnArgs, int) {
+  if (d == 64) return attn_dec_kernel<KT, 64, CTX>;
+  if (d == 128) return attn_dec_kernel<KT, 128, CTX>;
+  if (d == 256) return attn_dec_kernel<KT, 256, CTX>;
+  return nullptr;
+}
+}  // namespace
+
+void (*attn_dec_pick(int kt, int d, bool ctx))(AttnArgs, int) {
+  switch (kt) {
+    case MTP_F32: return ctx ? dec_pick<MTP_F32, true>(d) : dec_pick<MTP_F32, false>(d);
+    case MTP_BF16: return ctx ? dec_pick<MTP_BF16, true>(d) : dec_pick<MTP_BF16, false>(d);
+    case MTP_F16: return ctx ? dec_pick<MTP_F16, true>(d) : dec_pick<MTP_F16, false>(d);
+    // fp8 K / V are dense only
+    case MTP_FP8E4M3: return ctx ? nullptr : dec_pick<MTP_FP8E4M3, false>(d);
+  }
+  return nullptr;
+}
 
 void (*attn_generic())(AttnArgs, int, int) { return attn_generic_kernel; }
 

@@ -418,9 +418,9 @@ attn_merge_kernel(const AttnArgs a) {
   attn_store4<CT>(a, b, q, h, d4 * 4, O, 1.f / L);
 }
 
-// Fallback for shapes the MFMA kernel does not take (fp32 q / k / v, head
-// dims other than 64 / 128, more than 64 queries): one wave per (b, query,
-// h), keys in order, lanes split d. Same semantics and key sources.
+// Fallback for what neither the MFMA kernels nor the decode kernel
+// (attn_dec.hpp) take (head dims other than 64, 128, 256 and rows that are
+// not 16-byte aligned): one wave per (b, query, h), keys in order, lanes split d. Same semantics and key sources.
 __device__ __forceinline__ float load_kv_f32(const void *p, int dt, int64_t i) {
   if (dt == MTP_FP8E4M3) return __builtin_amdgcn_cvt_f32_fp8((uint32_t)((const uint8_t *)p)[i], 0);
   return load_as_f32(p, dt, i);

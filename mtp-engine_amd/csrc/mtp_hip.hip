@@ -32,7 +32,7 @@ std::once_flag g_tune_once;
 const char *const kTuneNames[kTuneCount] = {
     "skl", "sk_splits", "ws_variant", "ws_splits", "skl_waves", "skl_splits",
     "attn_chunk_blocks", "int4_waves", "verify_wstream", "skp", "skp_splits", "skp_ta", "sf32", "skp_h8", "attn32", "sk_xraw",
-    "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw"};
+    "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw", "attn_dec"};
 
 int env_int(const char *name, int dflt) {
   const char *e = std::getenv(name);
@@ -72,6 +72,7 @@ void tune_init() {
   g_tune[kTuneSklTw].store(env_int("MTP_SKL_TW", -1), std::memory_order_relaxed);
   g_tune[kTuneSkvR8].store(env_int("MTP_SKV_R8", -1), std::memory_order_relaxed);
   g_tune[kTuneSkvTw].store(env_int("MTP_SKV_TW", -1), std::memory_order_relaxed);
+  g_tune[kTuneAttnDec].store(env_int("MTP_ATTN_DEC", -1), std::memory_order_relaxed);
 }
 }  // namespace
 
@@ -1060,6 +1061,78 @@ AttnPlan make_attn_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int
   return p;
 }
 
+// Decode plan (attn_dec.hpp): head dims 64, 128 and 256 with one query per
+// (batch, head), and the shapes the MFMA kernels do not take (fp32, fp8 K / V,
+// more than 64 queries). A workgroup of `waves` waves takes chunk_blocks
+// blocks of 64 keys of one (batch, head, query).
+struct DecPlan {
+  bool fast = false;
+  int waves = 16, nchunks = 1, chunk_blocks = 1;
+  size_t part_off = 0, total = 0;
+};
+
+// What a merge of chunks costs (partials through the device coherence point,
+// arrival ticket, the last workgroup's loads), in blocks of 64 keys at the
+// rate a CU reads them when the whole chip reads (about 1.2 us for bf16 at
+// D 128), once and per chunk. bf16, D 128, L 4096, us per call: 8 heads 49.7
+// in one chunk, 19.5 in 4, 14.4 in 8, 11.3 in 16, 12.2 in 32; 256 heads 86.0
+// in one chunk, 100.1 in 4.
+constexpr double kDecMergeBlocks = 2.5, kDecMergeChunk = 0.2;
+
+DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64_t Lc, int64_t Lt,
+                      bool kv_fp8) {
+  DecPlan p;
+  if (D != 64 && D != 128 && D != 256) return p;
+  const bool mfma = (ct == MTP_BF16 || ct == MTP_F16) && D != 256 && NQ > 1 && NQ <= 64 && !kv_fp8;
+  if (mfma || tune(kTuneAttnDec) == 0) return p;
+  p.fast = true;
+  const int64_t units = B * H * NQ;
+  const int64_t blocks = (Lc + Lt + kAttnBlock - 1) / kAttnBlock;
+  if (blocks == 0) return p;
+  // 16 waves per CU in all: the workgroup size and chunk count with the
+  // least work on the busiest CU
+  const int maxw = dec_max_waves(kv_fp8 ? MTP_FP8E4M3 : ct);
+  double best = 0;
+  for (int nw = maxw; nw >= 4; nw /= 2) {
+    const int64_t slots = (int64_t)device_cus() * maxw / nw;
+    for (int64_t div : {1, 2, 4, 0}) {
+      int64_t nc = div ? slots / (units * div) : 1;
+      nc = std::max<int64_t>(1, std::min<int64_t>({nc, blocks, (int64_t)kAttnMaxChunks}));
+      int64_t cb = (blocks + nc - 1) / nc;
+      if (tune(kTuneAttnChunkBlocks) > 0) cb = std::min<int64_t>(tune(kTuneAttnChunkBlocks), blocks);
+      nc = (blocks + cb - 1) / cb;
+      if (nc > 1 && units > kCounterSlots) {
+        nc = 1;
+        cb = blocks;
+      }
+      // a workgroup's time: its blocks at its share of the CU, or at what
+      // its own waves can pull where the chip is not full
+      const int64_t rounds = (units * nc + slots - 1) / slots;
+      const double cost = (double)(rounds * cb) * maxw / nw +
+                          (nc > 1 ? kDecMergeBlocks + kDecMergeChunk * nc : 0);
+      if (best == 0 || cost < best) {
+        best = cost;
+        p.waves = nw;
+        p.nchunks = (int)nc;
+        p.chunk_blocks = (int)cb;
+      }
+    }
+  }
+  if (p.nchunks > 1) {
+    p.part_off = kCounterBytes;
+    p.total = kCounterBytes + align_up((size_t)units * p.nchunks * (D + 2) * 4, 256);
+  }
+  return p;
+}
+
+// Workspace of an attention call: the kernel it takes, or the largest
+// where several exist for the shape (fp8 or 16-bit K / V).
+size_t attn_ws_bytes(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64_t Lc, int64_t Lt) {
+  return std::max({make_attn_plan(ct, B, NQ, H, D, Lc, Lt).total,
+                   make_dec_plan(ct, B, NQ, H, D, Lc, Lt, false).total,
+                   make_dec_plan(ct, B, NQ, H, D, Lc, Lt, true).total});
+}
+
 // The 32-query-tile kernel takes 33 .. 64 queries at head dim 128 when its
 // buffer descriptors cover the key sources: every valid context row lies in
 // [0, npages * page stride) of the pages and the dense rows of a head span
@@ -1092,6 +1165,34 @@ int launch_attention(AttnArgs &a, int ct, int64_t D, void *ws, size_t ws_bytes, 
   const bool aligned = aligned16(a.q) && aligned16(a.out) && (!a.kp || aligned16(a.kp)) &&
                        (!a.vp || aligned16(a.vp)) && (!a.kd || aligned16(a.kd)) &&
                        (!a.vd || aligned16(a.vd));
+  DecPlan dp = make_dec_plan(ct, a.B, a.NQ, a.H, D, a.Lc, a.Lt, a.kv_fp8 != 0);
+  const int kt = a.kv_fp8 ? MTP_FP8E4M3 : ct;
+  // whole 16-byte pieces of every key row
+  const int kvec = 16 / dtype_bytes(kt);
+  const bool dec_rows = (a.p_sp | a.p_sb | a.p_sh | a.d_sb | a.d_sh | a.d_st) % kvec == 0 &&
+                        (!a.kp || aligned16(a.kp)) && (!a.vp || aligned16(a.vp)) &&
+                        (!a.kd || aligned16(a.kd)) && (!a.vd || aligned16(a.vd));
+  auto dk = dp.fast && dec_rows ? attn_dec_pick(kt, (int)D, a.Lc > 0) : nullptr;
+  if (dk) {
+    const size_t need = std::max(p.total, dp.total);
+    if (need > 0 && (!ws || ws_bytes < need)) {
+      // 16-bit calls need their workspace; the others took none before the
+      // chunks and still run without it, one workgroup per query
+      if (p.fast && !a.kv_fp8) return MTP_ERR_WORKSPACE;
+      dp.nchunks = 1;
+      dp.chunk_blocks = (int)((a.Lc + (int64_t)a.Lt + kAttnBlock - 1) / kAttnBlock);
+      dp.waves = dec_max_waves(kt);
+    }
+    a.nchunks = dp.nchunks;
+    a.chunk_blocks = dp.chunk_blocks;
+    if (dp.nchunks > 1) {
+      a.part = (float *)((unsigned char *)ws + dp.part_off);
+      a.ticket = (unsigned *)ws;
+    }
+    hipLaunchKernelGGL(dk, dim3((unsigned)(a.B * a.H), (unsigned)dp.nchunks, (unsigned)a.NQ),
+                       dim3((unsigned)(64 * dp.waves)), 0, st, a, ct);
+    return launch_status();
+  }
   if (p.fast && strides8 && aligned && !a.kv_fp8) {
     if (p.total > 0 && (!ws || ws_bytes < p.total)) return MTP_ERR_WORKSPACE;
     AttnKernel k = attn_pick(ct, (int)D);
@@ -1611,7 +1712,7 @@ int mtp_fused_multi_verify_textbook(const void *hidden, int h_dtype, int64_t B, 
 size_t mtp_attention_workspace_bytes(int dtype, int64_t B, int64_t NQ, int64_t H, int64_t D,
                                      int64_t Lc, int64_t Lt) {
   if (B <= 0 || NQ <= 0 || H <= 0 || D <= 0 || Lc < 0 || Lt < 0) return 0;
-  return make_attn_plan(dtype, B, NQ, H, D, Lc, Lt).total;
+  return attn_ws_bytes(dtype, B, NQ, H, D, Lc, Lt);
 }
 
 int mtp_fused_paged_attention(const void *q, int dtype, int64_t B, int64_t H, int64_t D,
@@ -1711,9 +1812,19 @@ int mtp_fused_causal_attention_fp8(const void *q, int dtype, int64_t B, int64_t 
                                    const float *kscale, const float *vscale, float scale,
                                    void *out, void *stream) {
   if (B > 0 && H > 0 && (!kscale || !vscale)) return MTP_ERR_NULL;
-  // the fp8 fallback kernel needs no workspace
+  // no workspace: the keys of a (batch, head) stay in one workgroup
   return dense_attention(q, dtype, B, H, D, k_fp8, v_fp8, L, nullptr, 0, 1, kscale, vscale, scale,
                          out, nullptr, 0, stream);
+}
+
+int mtp_fused_causal_attention_fp8_ws(const void *q, int dtype, int64_t B, int64_t H, int64_t D,
+                                      const void *k_fp8, const void *v_fp8, int64_t L,
+                                      const float *kscale, const float *vscale, float scale,
+                                      void *out, void *workspace, size_t workspace_bytes,
+                                      void *stream) {
+  if (B > 0 && H > 0 && (!kscale || !vscale)) return MTP_ERR_NULL;
+  return dense_attention(q, dtype, B, H, D, k_fp8, v_fp8, L, nullptr, 0, 1, kscale, vscale, scale,
+                         out, workspace, workspace_bytes, stream);
 }
 
 // Tree monolith: attention over the masked keys into an intermediate
@@ -1721,7 +1832,7 @@ int mtp_fused_causal_attention_fp8(const void *q, int dtype, int64_t B, int64_t 
 // head dimension (gamma rms_w) and the projection onto proj_w's rows.
 static size_t monolith_tmp_off(int dtype, int64_t B, int64_t H, int64_t D, int64_t L, int w_kind,
                                int64_t N) {
-  const size_t att = make_attn_plan(dtype, B, 1, H, D, 0, L).total;
+  const size_t att = attn_ws_bytes(dtype, B, 1, H, D, 0, L);
   const size_t lin = mtp_rmsnorm_linear_workspace_bytes(dtype, w_kind, B * H, N, D);
   return align_up(std::max(kCounterBytes, std::max(att, lin)), 256);
 }

@@ -77,6 +77,8 @@ SIGNATURES = {
         _i, [_vp, _i, _i64, _i64, _i64, _vp, _vp, _i64, _f, _vp, _vp, _sz, _vp]),
     "mtp_fused_causal_attention_fp8": (
         _i, [_vp, _i, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _f, _vp, _vp]),
+    "mtp_fused_causal_attention_fp8_ws": (
+        _i, [_vp, _i, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _f, _vp, _vp, _sz, _vp]),
     "mtp_fused_tree_attn_rmsnorm_linear": (
         _i, [_vp, _i, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _i, _vp, _i, _i64, _vp, _i, _vp, _i,
              _vp, _f, _f, _vp, _vp, _sz, _vp]),
@@ -155,7 +157,7 @@ def check(status: int, what: str) -> None:
 TUNING_KEYS = ("skl", "sk_splits", "ws_variant", "ws_splits", "skl_waves", "skl_splits",
                "attn_chunk_blocks", "int4_waves", "verify_wstream", "skp", "skp_splits",
                "skp_ta", "sf32", "skp_h8", "attn32", "sk_xraw",
-               "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw")
+               "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw", "attn_dec")
 
 
 def set_tuning(**keys: int) -> None:

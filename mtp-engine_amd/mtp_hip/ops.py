@@ -527,9 +527,12 @@ def causal_attention_fp8(q: torch.Tensor, k_fp8: torch.Tensor, v_fp8: torch.Tens
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     out = torch.empty_like(q)
-    s = lib.mtp_fused_causal_attention_fp8(ptr(q), code(q.dtype), B, H, D, ptr(k_fp8),
-                                           ptr(v_fp8), L, ptr(kscale), ptr(vscale), float(scale),
-                                           ptr(out), _lib.stream_handle(q.device))
+    nbytes = lib.mtp_attention_workspace_bytes(code(q.dtype), B, 1, H, D, 0, L)
+    ws = _lib.workspace(q.device, nbytes)
+    s = lib.mtp_fused_causal_attention_fp8_ws(ptr(q), code(q.dtype), B, H, D, ptr(k_fp8),
+                                              ptr(v_fp8), L, ptr(kscale), ptr(vscale),
+                                              float(scale), ptr(out), ptr(ws), nbytes,
+                                              _lib.stream_handle(q.device))
     check(s, "fused_causal_attention_fp8")
     return out
 

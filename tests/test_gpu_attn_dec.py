@@ -1,0 +1,165 @@
+"""Decode attention kernel (one query per batch row and head; fp32, 16-bit
+and fp8 K / V) against the oracle and against the kernels it replaces, where
+it can go wrong: key counts around a step (8 .. 64 keys), a block (64) and a
+chunk, every row width, chunked and whole contexts, both key sources, masks
+of every dtype, rows with no key. Bound |y - ref| <= rtol (|ref| + RMS(ref)):
+fp32 1e-5 (sums of up to some thousand fp32 terms and exp of fp32 scores),
+16-bit outputs 2e-2 (the oracle rounds probabilities to the type)."""
+import pytest
+import torch
+
+from conftest import close
+from oracle import eager as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+RTOL = {torch.bfloat16: 2e-2, torch.float16: 2e-2, torch.float32: 1e-5}
+
+
+def _check(out, ref, dtype):
+    assert torch.equal(torch.isnan(out.cpu()), torch.isnan(ref.cpu()))
+    ok, worst = close(torch.nan_to_num(out.cpu()), torch.nan_to_num(ref.cpu()), RTOL[dtype])
+    assert ok, f"worst err/bound = {worst:.3g}"
+
+
+@pytest.mark.parametrize("chunk_blocks", [-1, 1, 3])
+@pytest.mark.parametrize("dtype,kv", [(torch.float32, "same"), (torch.bfloat16, "same"),
+                                      (torch.float16, "same"), (torch.float32, "fp8"),
+                                      (torch.bfloat16, "fp8"), (torch.float16, "fp8")])
+@pytest.mark.parametrize("B,H,L,D", [(1, 1, 1, 64), (2, 3, 63, 256), (1, 2, 65, 64),
+                                     (3, 1, 129, 128), (2, 2, 1601, 128), (1, 2, 4097, 64)])
+def test_dense(B, H, L, D, dtype, kv, chunk_blocks, tune):
+    import mtp_kernels as mk
+    tune(attn_chunk_blocks=chunk_blocks)
+    g = torch.Generator().manual_seed(B * L + D)
+    q = torch.randn(B, H, D, generator=g).to(dtype)
+    k, v = torch.randn(B, H, L, D, generator=g), torch.randn(B, H, L, D, generator=g)
+    print(f"case decode dense {dtype} {kv} B={B} H={H} L={L} D={D} cb={chunk_blocks}", flush=True)
+    if kv == "fp8":
+        ks, vs = 0.01 + 0.01 * torch.rand(H, generator=g), 0.01 + 0.01 * torch.rand(H, generator=g)
+        k = (k / ks[None, :, None, None]).to(torch.float8_e4m3fn)
+        v = (v / vs[None, :, None, None]).to(torch.float8_e4m3fn)
+        ref = O.causal_attention_fp8(q, k, v, ks, vs)
+        args = [t.to(DEV) for t in (q, k, v, ks, vs)]
+        out = mk.fused_causal_attention_fp8(*args)
+    else:
+        k, v = k.to(dtype), v.to(dtype)
+        ref = O.causal_attention(q, k, v)
+        args = [t.to(DEV) for t in (q, k, v)]
+        out = mk.fused_causal_attention(*args)
+    _check(out, ref, dtype)
+    # the kernel of every other shape gives the same within the bound
+    tune(attn_dec=0)
+    old = (mk.fused_causal_attention_fp8 if kv == "fp8" else mk.fused_causal_attention)(*args)
+    _check(out, old, dtype)
+
+
+@pytest.mark.parametrize("mdtype", [torch.float32, torch.bfloat16, torch.float16, torch.bool,
+                                    torch.uint8])
+@pytest.mark.parametrize("dtype,D,L", [(torch.float32, 64, 300), (torch.float32, 128, 64),
+                                       (torch.bfloat16, 256, 77), (torch.float16, 128, 500)])
+def test_masks(dtype, D, L, mdtype, tune):
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(L)
+    B, H = 2, 3
+    q = torch.randn(B, H, D, generator=g).to(dtype)
+    k = torch.randn(B, H, L, D, generator=g).to(dtype)
+    v = torch.randn(B, H, L, D, generator=g).to(dtype)
+    for mask in (torch.rand(L, generator=g) > 0.9, torch.zeros(L, dtype=torch.bool),
+                 torch.arange(L) == L - 1):
+        m = mask.to(mdtype)
+        for cb in (-1, 1):
+            tune(attn_chunk_blocks=cb)
+            print(f"case decode mask {dtype} {mdtype} D={D} L={L} cb={cb}", flush=True)
+            out = mk.fused_tree_attention(q.to(DEV), k.to(DEV), v.to(DEV), m.to(DEV))
+            _check(out, O.tree_attention(q, k, v, mask.float()), dtype)
+
+
+@pytest.mark.parametrize("dtype,B,H,L,D,ps", [(torch.bfloat16, 2, 3, 130, 128, 16),
+                                              (torch.float16, 1, 2, 777, 64, 5),
+                                              (torch.float32, 3, 2, 1100, 128, 32),
+                                              (torch.bfloat16, 2, 2, 64, 256, 7)])
+def test_paged(dtype, B, H, L, D, ps, tune):
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(L + ps)
+    n = -(-L // ps)
+    P = n + 2
+    q = torch.randn(B, H, D, generator=g).to(dtype)
+    kp = torch.randn(P, B, H, ps, D, generator=g).to(dtype)
+    vp = torch.randn(P, B, H, ps, D, generator=g).to(dtype)
+    table = torch.stack([torch.randperm(P, generator=g)[:n].repeat_interleave(ps)[:L]
+                         for _ in range(B)]).to(torch.int32)
+    ref = O.paged_attention(q, kp, vp, table, ps)
+    args = [t.to(DEV) for t in (q, kp, vp, table)]
+    for cb in (-1, 1, 4):
+        tune(attn_chunk_blocks=cb)
+        print(f"case decode paged {dtype} L={L} D={D} ps={ps} cb={cb}", flush=True)
+        _check(mk.fused_paged_attention(*args, ps), ref, dtype)
+    # pages outside the cache are keys that are not there
+    bad = table.clone()
+    bad[:, ::3] = -1
+    bad[0, 1::3] = P
+    out = mk.fused_paged_attention(q.to(DEV), kp.to(DEV), vp.to(DEV), bad.to(DEV), ps)
+    tune(attn_dec=0)
+    _check(out, mk.fused_paged_attention(q.to(DEV), kp.to(DEV), vp.to(DEV), bad.to(DEV), ps), dtype)
+
+
+@pytest.mark.parametrize("N,H,Lc,D", [(5, 2, 100, 128), (70, 2, 65, 64), (3, 4, 0, 64)])
+def test_tree_verify_fp32(N, H, Lc, D, tune):
+    """Several fp32 queries per head over both key sources and a 2-D mask."""
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(N)
+    ps, n = 16, -(-Lc // 16)
+    q, kt, vt = (torch.randn(N, H, D, generator=g) for _ in range(3))
+    kp, vp = (torch.randn(n + 1, 1, H, ps, D, generator=g) for _ in range(2))
+    table = torch.randperm(n + 1, generator=g)[:n].repeat_interleave(ps)[:Lc].to(torch.int32)[None]
+    tm = torch.tril((torch.rand(N, N, generator=g) > 0.5).float())
+    tm.fill_diagonal_(1.0)
+    ref = O.tree_verify_attention(q, kp, vp, table, ps, kt, vt, tm)
+    for cb in (-1, 1):
+        tune(attn_chunk_blocks=cb)
+        print(f"case decode tree-verify fp32 N={N} H={H} Lc={Lc} D={D} cb={cb}", flush=True)
+        out = mk.tree_verify_attention(*(t.to(DEV) for t in (q, kp, vp, table)), ps,
+                                       *(t.to(DEV) for t in (kt, vt, tm)))
+        _check(out, ref, torch.float32)
+
+
+def test_infinite_and_nan_scores():
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(1)
+    q = torch.randn(1, 1, 64, generator=g)
+    k = torch.randn(1, 1, 200, 64, generator=g)
+    v = torch.randn(1, 1, 200, 64, generator=g)
+    for val in (float("inf"), float("nan"), -1e38):
+        k2 = k.clone()
+        k2[0, 0, 150, 3] = val
+        out = mk.fused_causal_attention(q.to(DEV), k2.to(DEV), v.to(DEV))
+        _check(out, O.causal_attention(q, k2, v), torch.float32)
+
+
+def test_unaligned_rows_take_the_general_kernel():
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(2)
+    q = torch.randn(1, 2, 64, generator=g)
+    buf = torch.randn(2 * 50 * 64 + 1, generator=g).to(DEV)
+    k = buf[1:].view(1, 2, 50, 64)
+    out = mk.fused_causal_attention(q.to(DEV), k, k)
+    _check(out, O.causal_attention(q, k.cpu(), k.cpu()), torch.float32)
+
+
+def test_fp8_entry_without_workspace():
+    """The C entry that takes no workspace reads every key in one workgroup."""
+    from mtp_hip import _lib as L
+    from mtp_hip import ops
+    g = torch.Generator().manual_seed(4)
+    B, H, N, D = 1, 2, 1000, 128
+    q = torch.randn(B, H, D, generator=g).to(torch.bfloat16).to(DEV)
+    k = torch.randn(B, H, N, D, generator=g).to(torch.float8_e4m3fn).to(DEV)
+    v = torch.randn(B, H, N, D, generator=g).to(torch.float8_e4m3fn).to(DEV)
+    s = torch.ones(H, device=DEV)
+    out = torch.empty_like(q)
+    st = L.load().mtp_fused_causal_attention_fp8(
+        q.data_ptr(), L.BF16, B, H, D, k.data_ptr(), v.data_ptr(), N, s.data_ptr(), s.data_ptr(),
+        D ** -0.5, out.data_ptr(), L.stream_handle(q.device))
+    assert st == L.OK
+    _check(out, ops.causal_attention_fp8(q, k, v, s, s), torch.bfloat16)
