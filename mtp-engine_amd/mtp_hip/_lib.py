@@ -193,8 +193,18 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The current stream's handle by device index, without the Stream object that
+# torch.cuda.current_stream() makes on every call (1.8 us against 0.1, twice a
+# call).
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def _index(device: torch.device) -> int:
+    return torch.cuda.current_device() if device.index is None else device.index
+
+
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(_index(device))
 
 
 # ---------------------------------------------------------------------------
@@ -231,7 +241,7 @@ def _grown(ws, nbytes: int) -> int:
 def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
     if nbytes == 0:
         return None
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (_index(device), stream_handle(device))
     ws = _workspaces.get(key)
     if ws is not None and ws.numel() >= nbytes:
         return ws
@@ -248,6 +258,19 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
     ws = _new_workspace(device, _grown(ws, nbytes))
     _workspaces[key] = ws
     return ws
+
+
+def scratch(t: torch.Tensor, nbytes: int):
+    """(workspace address or None, current stream handle) for a call on t's
+    device."""
+    idx = t.get_device()
+    st = _raw_stream(idx)
+    if nbytes == 0:
+        return None, st
+    ws = _workspaces.get((idx, st))
+    if ws is None or ws.numel() < nbytes:
+        ws = workspace(t.device, nbytes)
+    return ws.data_ptr(), st
 
 
 def reserve_workspace(device: torch.device, nbytes: int, stream=None) -> torch.Tensor:

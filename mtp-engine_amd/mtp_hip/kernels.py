@@ -78,7 +78,7 @@ def fused_rmsnorm_linear(
     the reference does (line 952)."""
     if scale is None:
         scale = TUNING.fp8_scale
-    if bias is not None:
+    if bias is not None and (bias.dtype is not x.dtype or bias.device != x.device):
         bias = bias.to(dtype=x.dtype, device=x.device)
     return ops.rmsnorm_linear(x, weight, bias, eps, scale, gamma=gamma, norm=norm)
 

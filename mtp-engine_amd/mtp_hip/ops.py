@@ -22,11 +22,20 @@ _FLOATS = (torch.float32, torch.bfloat16, torch.float16)
 def _on_device(name: str, t: torch.Tensor, **others) -> None:
     """Every tensor handed to the library must live on the same HIP device:
     a host tensor's data_ptr() is not a device address."""
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise RuntimeError(f"mtp_hip: {name} must be on a HIP device (got {t.device})")
+    d = t.get_device()
     for k, o in others.items():
-        if o is not None and o.device != t.device:
+        if o is not None and o.get_device() != d:
             raise RuntimeError(f"mtp_hip: {k} is on {o.device}, expected {t.device} like {name}")
+
+
+def _f32(t: torch.Tensor) -> torch.Tensor:
+    return t if t.dtype is torch.float32 else t.to(torch.float32)
+
+
+def _i32(t: torch.Tensor) -> torch.Tensor:
+    return t if t.dtype is torch.int32 else t.to(torch.int32)
 
 
 def rmsnorm_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -44,18 +53,17 @@ def rmsnorm_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
         bias = bias.contiguous()
         assert bias.numel() == N, f"fused_rmsnorm_linear: bias has {bias.numel()} != {N}"
     if gamma is not None:
-        gamma = gamma.contiguous().to(torch.float32)
+        gamma = _f32(gamma.contiguous())
         assert gamma.numel() == K, f"fused_rmsnorm_linear: gamma has {gamma.numel()} != {K}"
     _on_device("x", x, weight=weight, bias=bias, gamma=gamma)
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    y = x.new_empty((M, N))
     nbytes = lib.mtp_rmsnorm_linear_workspace_bytes(code(x.dtype), code(weight.dtype), M, N, K)
-    ws = _lib.workspace(x.device, nbytes)
+    ws, stream = _lib.scratch(x, nbytes)
     st = lib.mtp_fused_rmsnorm_linear(
         ptr(x), code(x.dtype), M, K, ptr(weight), code(weight.dtype), N,
         ptr(bias), code(bias.dtype) if bias is not None else 0,
         ptr(gamma), code(gamma.dtype) if gamma is not None else 0,
-        float(eps), float(scale), int(bool(norm)), ptr(y), ptr(ws), nbytes,
-        _lib.stream_handle(x.device))
+        float(eps), float(scale), int(bool(norm)), ptr(y), ws, nbytes, stream)
     check(st, "fused_rmsnorm_linear")
     return y
 
@@ -67,7 +75,7 @@ def rmsnorm_linear_fp8(x: torch.Tensor, weight_fp8: torch.Tensor, wscale: torch.
     lib = _lib.load()
     x = x.contiguous()
     weight_fp8 = weight_fp8.contiguous()
-    wscale = wscale.contiguous().to(torch.float32)
+    wscale = _f32(wscale.contiguous())
     assert x.dim() == 2 and weight_fp8.dim() == 2, "fused_rmsnorm_linear_fp8: 2-D x and weight"
     M, K = x.shape
     N, K2 = weight_fp8.shape
@@ -77,20 +85,20 @@ def rmsnorm_linear_fp8(x: torch.Tensor, weight_fp8: torch.Tensor, wscale: torch.
         bias = bias.contiguous()
         assert bias.numel() == N, f"fused_rmsnorm_linear_fp8: bias has {bias.numel()} != {N}"
     if gamma is not None:
-        gamma = gamma.contiguous().to(torch.float32)
+        gamma = _f32(gamma.contiguous())
         assert gamma.numel() == K, f"fused_rmsnorm_linear_fp8: gamma has {gamma.numel()} != {K}"
     _on_device("x", x, weight=weight_fp8, wscale=wscale, bias=bias, gamma=gamma)
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    y = x.new_empty((M, N))
     # The reference accepts any weight dtype here (its self-test passes fp32
     # values in +-448); the library takes the weight dtype as given.
     wcode = code(weight_fp8.dtype)
     nbytes = lib.mtp_rmsnorm_linear_workspace_bytes(code(x.dtype), wcode, M, N, K)
-    ws = _lib.workspace(x.device, nbytes)
+    ws, stream = _lib.scratch(x, nbytes)
     st = lib.mtp_fused_rmsnorm_linear_fp8(
         ptr(x), code(x.dtype), M, K, ptr(weight_fp8), wcode, ptr(wscale), N,
         ptr(bias), code(bias.dtype) if bias is not None else 0,
         ptr(gamma), code(gamma.dtype) if gamma is not None else 0,
-        float(eps), int(bool(norm)), ptr(y), ptr(ws), nbytes, _lib.stream_handle(x.device))
+        float(eps), int(bool(norm)), ptr(y), ws, nbytes, stream)
     check(st, "fused_rmsnorm_linear_fp8")
     return y
 
@@ -118,13 +126,13 @@ def int4_matmul(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, K: 
     _on_device("x", x, packed=packed, scales=scales, gamma=gamma)
     mode = {"ref": _lib.NIBBLE_OFFSET8, "offset": _lib.NIBBLE_OFFSET8,
             "twos": _lib.NIBBLE_TWOS}[nibble]
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    y = x.new_empty((M, N))
     nbytes = lib.mtp_rmsnorm_linear_workspace_bytes(code(x.dtype), _lib.U8, M, N, K)
-    ws = _lib.workspace(x.device, nbytes)
+    ws, stream = _lib.scratch(x, nbytes)
     st = lib.mtp_fused_int4_matmul(
         ptr(x), code(x.dtype), M, K, ptr(packed), ptr(scales), code(scales.dtype), N, int(group),
         mode, ptr(gamma), code(gamma.dtype) if gamma is not None else 0, float(eps),
-        int(bool(norm)), ptr(y), ptr(ws), nbytes, _lib.stream_handle(x.device))
+        int(bool(norm)), ptr(y), ws, nbytes, stream)
     check(st, "fused_int4_matmul")
     return y
 
@@ -135,7 +143,7 @@ def verify(hidden: torch.Tensor, weight: torch.Tensor, draft: torch.Tensor,
     lib = _lib.load()
     hidden = hidden.contiguous()
     weight = weight.contiguous()
-    draft = draft.contiguous().to(torch.int32)
+    draft = _i32(draft.contiguous())
     assert hidden.dim() == 2 and weight.dim() == 2, "fused_verify: 2-D hidden and weight"
     M, K = hidden.shape
     V = weight.shape[0]
@@ -148,11 +156,11 @@ def verify(hidden: torch.Tensor, weight: torch.Tensor, draft: torch.Tensor,
     accept = torch.empty(M, dtype=torch.int8, device=hidden.device)
     top = torch.empty(M, dtype=torch.int32, device=hidden.device)
     nbytes = lib.mtp_verify_workspace_bytes(code(hidden.dtype), M, 1, V, K)
-    ws = _lib.workspace(hidden.device, nbytes)
+    ws, stream = _lib.scratch(hidden, nbytes)
     st = lib.mtp_fused_verify(
         ptr(hidden), code(hidden.dtype), M, K, ptr(weight), code(weight.dtype), V,
         ptr(bias), code(bias.dtype) if bias is not None else 0, ptr(draft), ptr(accept), ptr(top),
-        ptr(ws), nbytes, _lib.stream_handle(hidden.device))
+        ws, nbytes, stream)
     check(st, "fused_verify")
     return accept, top
 
@@ -191,7 +199,7 @@ def multi_verify(hidden: torch.Tensor, weight: torch.Tensor, draft: torch.Tensor
     lib = _lib.load()
     hidden = hidden.contiguous()
     weight = weight.contiguous()
-    draft = draft.contiguous().to(torch.int32)
+    draft = _i32(draft.contiguous())
     assert hidden.dim() == 3 and weight.dim() == 2 and draft.dim() == 2, \
         "fused_multi_verify: hidden [B, S, K], weight [V, K], draft [B, D]"
     B, S, K = hidden.shape
@@ -210,13 +218,13 @@ def multi_verify(hidden: torch.Tensor, weight: torch.Tensor, draft: torch.Tensor
     corrected = torch.empty((B,), dtype=torch.int32, device=dev)
     top = torch.empty((B, S), dtype=torch.int32, device=dev) if return_top else None
     nbytes = lib.mtp_verify_workspace_bytes(code(hidden.dtype), B * S, S, V, K)
-    ws = _lib.workspace(dev, nbytes)
+    ws, stream = _lib.scratch(hidden, nbytes)
     fn = lib.mtp_fused_multi_verify if convention == "reference" else \
         lib.mtp_fused_multi_verify_textbook
     st = fn(
         ptr(hidden), code(hidden.dtype), B, S, K, ptr(weight), code(weight.dtype), V,
         ptr(bias), code(bias.dtype) if bias is not None else 0, ptr(draft), D, ptr(accept),
-        ptr(accepted_n), ptr(corrected), ptr(top), ptr(ws), nbytes, _lib.stream_handle(dev))
+        ptr(accepted_n), ptr(corrected), ptr(top), ws, nbytes, stream)
     check(st, "fused_multi_verify")
     if return_top:
         return accept, accepted_n, corrected, top
@@ -236,8 +244,8 @@ def _attn_call(fn_name: str, q: torch.Tensor, B: int, NQ: int, H: int, D: int, L
                *args) -> None:
     lib = _lib.load()
     nbytes = lib.mtp_attention_workspace_bytes(code(q.dtype), B, NQ, H, D, Lc, Lt)
-    ws = _lib.workspace(q.device, nbytes)
-    st = getattr(lib, fn_name)(*args, ptr(ws), nbytes, _lib.stream_handle(q.device))
+    ws, stream = _lib.scratch(q, nbytes)
+    st = getattr(lib, fn_name)(*args, ws, nbytes, stream)
     check(st, fn_name[4:])
 
 
@@ -247,7 +255,7 @@ def paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tenso
     q = q.contiguous()
     k_pages = k_pages.contiguous()
     v_pages = v_pages.contiguous()
-    page_table = page_table.contiguous().to(torch.int32)
+    page_table = _i32(page_table.contiguous())
     assert q.dim() == 3, "fused_paged_attention: q [B, H, D]"
     B, H, D = q.shape
     L = page_table.shape[-1]
@@ -303,7 +311,7 @@ def tree_verify_attention(q_nodes: torch.Tensor, k_pages: torch.Tensor, v_pages:
     v_tree = v_tree.contiguous()
     k_pages = k_pages.contiguous()
     v_pages = v_pages.contiguous()
-    page_table = page_table.contiguous().to(torch.int32)
+    page_table = _i32(page_table.contiguous())
     tree_mask = _mask_arg(tree_mask)
     assert q_nodes.dim() == 3, "tree_verify_attention: q_nodes [N, H, D]"
     N, H, D = q_nodes.shape
@@ -339,9 +347,8 @@ def quantize_fp8_tensor(x: torch.Tensor):
     n = x.numel()
     assert n > 0, "quantize_fp8_e4m3: empty tensor"
     nbytes = lib.mtp_quantize_workspace_bytes(n)
-    ws = _lib.workspace(x.device, nbytes)
-    st = lib.mtp_quantize_fp8_e4m3(ptr(x), code(x.dtype), n, ptr(q), ptr(scale), ptr(ws), nbytes,
-                                   _lib.stream_handle(x.device))
+    ws, stream = _lib.scratch(x, nbytes)
+    st = lib.mtp_quantize_fp8_e4m3(ptr(x), code(x.dtype), n, ptr(q), ptr(scale), ws, nbytes, stream)
     check(st, "quantize_fp8_e4m3")
     return q, scale
 
@@ -426,7 +433,9 @@ def rmsnorm(x: torch.Tensor, weight: Optional[torch.Tensor] = None, eps: float =
     assert x.dim() == 2, "fused_rmsnorm: x must be 2-D [M, N]"
     M, N = x.shape
     if weight is not None:
-        weight = weight.contiguous().to(dtype=x.dtype, device=x.device)
+        weight = weight.contiguous()
+        if weight.dtype is not x.dtype or weight.device != x.device:
+            weight = weight.to(dtype=x.dtype, device=x.device)
         assert weight.numel() == N, f"fused_rmsnorm: weight has {weight.numel()} != {N}"
     if residual is not None:
         residual = residual.contiguous()
@@ -468,12 +477,12 @@ def argmax(logits: torch.Tensor, emb_table: Optional[torch.Tensor] = None):
         assert emb_table.dim() == 2, "argmax: emb_table must be [V, H]"
         emb = torch.empty((M, emb_table.shape[1]), dtype=emb_table.dtype, device=lg.device)
     nbytes = lib.mtp_argmax_workspace_bytes(M, V)
-    ws = _lib.workspace(lg.device, nbytes)
+    ws, stream = _lib.scratch(lg, nbytes)
     s = lib.mtp_argmax(ptr(lg), code(lg.dtype), M, V, ld, ptr(tokens), ptr(emb_table),
                        code(emb_table.dtype) if emb_table is not None else 0,
                        emb_table.shape[0] if emb_table is not None else 0,
-                       emb_table.shape[1] if emb_table is not None else 0, ptr(emb), ptr(ws),
-                       nbytes, _lib.stream_handle(lg.device))
+                       emb_table.shape[1] if emb_table is not None else 0, ptr(emb), ws,
+                       nbytes, stream)
     check(s, "argmax")
     if one_d:
         tokens = tokens.reshape(())
@@ -499,10 +508,9 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         scale = 1.0 / math.sqrt(D)
     out = torch.empty_like(q)
     nbytes = lib.mtp_attention_workspace_bytes(code(q.dtype), B, 1, H, D, 0, L)
-    ws = _lib.workspace(q.device, nbytes)
+    ws, stream = _lib.scratch(q, nbytes)
     s = lib.mtp_fused_causal_attention(ptr(q), code(q.dtype), B, H, D, ptr(k), ptr(v), L,
-                                       float(scale), ptr(out), ptr(ws), nbytes,
-                                       _lib.stream_handle(q.device))
+                                       float(scale), ptr(out), ws, nbytes, stream)
     check(s, "fused_causal_attention")
     return out
 
@@ -514,8 +522,8 @@ def causal_attention_fp8(q: torch.Tensor, k_fp8: torch.Tensor, v_fp8: torch.Tens
     [H] / vscale [H]."""
     lib = _lib.load()
     q, k_fp8, v_fp8 = q.contiguous(), k_fp8.contiguous(), v_fp8.contiguous()
-    kscale = kscale.contiguous().to(torch.float32)
-    vscale = vscale.contiguous().to(torch.float32)
+    kscale = _f32(kscale.contiguous())
+    vscale = _f32(vscale.contiguous())
     B, H, D = q.shape
     _B, _H, L, _D = k_fp8.shape
     assert (B, H, D) == (_B, _H, _D)
@@ -528,11 +536,10 @@ def causal_attention_fp8(q: torch.Tensor, k_fp8: torch.Tensor, v_fp8: torch.Tens
         scale = 1.0 / math.sqrt(D)
     out = torch.empty_like(q)
     nbytes = lib.mtp_attention_workspace_bytes(code(q.dtype), B, 1, H, D, 0, L)
-    ws = _lib.workspace(q.device, nbytes)
+    ws, stream = _lib.scratch(q, nbytes)
     s = lib.mtp_fused_causal_attention_fp8_ws(ptr(q), code(q.dtype), B, H, D, ptr(k_fp8),
                                               ptr(v_fp8), L, ptr(kscale), ptr(vscale),
-                                              float(scale), ptr(out), ptr(ws), nbytes,
-                                              _lib.stream_handle(q.device))
+                                              float(scale), ptr(out), ws, nbytes, stream)
     check(s, "fused_causal_attention_fp8")
     return out
 
@@ -565,7 +572,7 @@ def tree_attn_rmsnorm_linear(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         proj_bias = proj_bias.contiguous()
         assert proj_bias.numel() == N
     if wscale is not None:
-        wscale = wscale.contiguous().to(torch.float32)
+        wscale = _f32(wscale.contiguous())
         assert wscale.numel() == N
     _on_device("q", q, k=k, v=v, mask=mask, proj_w=proj_w, rms_w=rms_w, proj_bias=proj_bias,
                wscale=wscale)
@@ -574,12 +581,12 @@ def tree_attn_rmsnorm_linear(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     out = torch.empty((B, H, N), dtype=q.dtype, device=q.device)
     wkind = _lib.FP8E4M3 if wscale is not None else code(proj_w.dtype)
     nbytes = lib.mtp_tree_attn_rmsnorm_linear_workspace_bytes(code(q.dtype), B, H, D, L, wkind, N)
-    ws = _lib.workspace(q.device, nbytes)
+    ws, stream = _lib.scratch(q, nbytes)
     s = lib.mtp_fused_tree_attn_rmsnorm_linear(
         ptr(q), code(q.dtype), B, H, D, ptr(k), ptr(v), L, ptr(mask), code(mask.dtype),
         ptr(proj_w), code(proj_w.dtype), N, ptr(rms_w), _lib.F32 if rms_w is not None else 0,
         ptr(proj_bias), code(proj_bias.dtype) if proj_bias is not None else 0, ptr(wscale),
-        float(scale), float(eps), ptr(out), ptr(ws), nbytes, _lib.stream_handle(q.device))
+        float(scale), float(eps), ptr(out), ws, nbytes, stream)
     check(s, "fused_tree_attn_rmsnorm_linear")
     return out
 
@@ -605,7 +612,7 @@ def paged_kv_write(k_new: torch.Tensor, v_new: torch.Tensor, k_pages: torch.Tens
         "paged_kv_write: pages must be contiguous [P, B, H, page_size, D]"
     P, _B, _H, ps, _D = k_pages.shape
     assert (_B, _H, _D) == (B, H, D), "paged_kv_write: pages do not match the new rows"
-    page_table = page_table.contiguous().to(torch.int32)
+    page_table = _i32(page_table.contiguous())
     assert page_table.dim() == 2 and page_table.shape[0] == B, "paged_kv_write: page_table [B, L]"
     start_dev, per_row, start_host = None, 0, 0
     if torch.is_tensor(start):
