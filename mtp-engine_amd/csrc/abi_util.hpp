@@ -64,6 +64,8 @@ enum TuneKey {
   kTuneSkvR8,            // MTP_SKV_R8: fp32 verify, 8 rows after whole 16-row tiles on the 4x4 MFMA (0: off)
   kTuneSkvTw,            // MTP_SKV_TW: streaming verify's columns per tile (8 .. 256, multiple of 8)
   kTuneAttnDec,          // MTP_ATTN_DEC: decode attention kernel, 0 off (MFMA / fallback kernels)
+  kTunePg,               // MTP_PG: prompt GEMM, 0 off, n > 0 forces tile shape n - 1
+  kTunePgSplits,         // MTP_PG_SPLITS: K-splits of its 4-wave shapes
   kTuneCount
 };
 int tune(TuneKey k);

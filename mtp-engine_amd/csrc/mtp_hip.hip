@@ -13,6 +13,7 @@
 #include "attn_args.hpp"
 #include "generic.hpp"
 #include "int4g_args.hpp"
+#include "pg_args.hpp"
 #include "quant.hpp"
 #include "sf32_args.hpp"
 #include "sk_args.hpp"
@@ -32,7 +33,7 @@ std::once_flag g_tune_once;
 const char *const kTuneNames[kTuneCount] = {
     "skl", "sk_splits", "ws_variant", "ws_splits", "skl_waves", "skl_splits",
     "attn_chunk_blocks", "int4_waves", "verify_wstream", "skp", "skp_splits", "skp_ta", "sf32", "skp_h8", "attn32", "sk_xraw",
-    "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw", "attn_dec"};
+    "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw", "attn_dec", "pg", "pg_splits"};
 
 int env_int(const char *name, int dflt) {
   const char *e = std::getenv(name);
@@ -72,6 +73,8 @@ void tune_init() {
   g_tune[kTuneSklTw].store(env_int("MTP_SKL_TW", -1), std::memory_order_relaxed);
   g_tune[kTuneSkvR8].store(env_int("MTP_SKV_R8", -1), std::memory_order_relaxed);
   g_tune[kTuneSkvTw].store(env_int("MTP_SKV_TW", -1), std::memory_order_relaxed);
+  g_tune[kTunePgSplits].store(env_int("MTP_PG_SPLITS", -1), std::memory_order_relaxed);
+  g_tune[kTunePg].store(env_int("MTP_PG", -1), std::memory_order_relaxed);
   g_tune[kTuneAttnDec].store(env_int("MTP_ATTN_DEC", -1), std::memory_order_relaxed);
 }
 }  // namespace
@@ -79,6 +82,13 @@ void tune_init() {
 int tune(TuneKey k) {
   std::call_once(g_tune_once, tune_init);
   return g_tune[k].load(std::memory_order_relaxed);
+}
+
+// Counts the changes of the tuning keys (plans kept by a thread end with it).
+std::atomic<unsigned> g_tune_epoch{1};
+unsigned tune_epoch() {
+  tune(kTuneSkl);  // the environment's keys first
+  return g_tune_epoch.load(std::memory_order_acquire);
 }
 
 int device_cus() {
@@ -830,6 +840,167 @@ int launch_skp(const PlanSkp &p, SkpArgs &a, void *ws, hipStream_t st) {
   return launch_status();
 }
 
+// ---------------------------------------------------------------------------
+// Prompt GEMM plan (pg.hpp): more than 64 rows of 16-bit x, W of fp8 or the
+// same 16-bit type, whole 64-k stages. Workspace: counters (left alone),
+// x * gamma (gamma only) and the row factors.
+struct PlanPg {
+  bool ok = false;
+  int ct = 0, wt = 0, shape = 0, S = 1, kper = 0, tiles = 0;
+  bool gam = false;
+  size_t xg_off = 0, rs_off = 0, part_off = 0, total = 0;
+};
+
+// Shape and K-splits by a model of the launch, in us: the longer of
+//  * the chain of stages of the busiest CU: the matrix instructions of a
+//    stage plus what its barrier and LDS round trips leave open (0.1 us, fp8
+//    0.16 with the upcast; 1.4 x with a second workgroup on the CU), and
+//  * the copies of all workgroups at the rate the L2s sustain (15 TB/s; 22
+//    while x and W together stay below 80 MB),
+// plus the hand-over of splits. Fitted to 32 sizes x 14 shapes, M 90 .. 2048,
+// N 600 .. 14336, K 512 .. 4096: its picks are 0 .. 12 % off the best shape.
+// bf16, us: 2048 x 14336 x 4096 on {7, 4} 200 (whole rounds of 256 tiles;
+// {8, 4} 203, {4, 4} 4-wave 272), 517 x 14336 on {6, 3} 67 ({8, 4} 92),
+// 128 x 1000 x 4096 on 4 splits of {2, 1} 13.0 (no split 16.6, {8, 4} 73).
+constexpr int64_t kPgSmallBytes = (int64_t)80 << 20;
+
+PlanPg plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
+  PlanPg p;
+  p.ct = ct;
+  p.wt = wt;
+  p.gam = gam;
+  if (ct != MTP_BF16 && ct != MTP_F16) return p;
+  if (wt != MTP_FP8E4M3 && wt != ct) return p;
+  if (tune(kTunePg) == 0 || M <= 64 || N <= 0 || K <= 0 || K % kPgK != 0) return p;
+  if (tune(kTuneWsVariant) >= 0 || tune(kTuneWsSplits) > 0) return p;  // sweeps of wsp
+  // buffer descriptors: a tile's rows of x and of W (256 at most)
+  if (256 * K * 2 >= (int64_t)1 << 31) return p;
+  const int wb = dtype_bytes(wt);
+  const int64_t steps = K / kPgK;
+  // copies of W and x that a pass over the chip's L2s sustains, bytes per us
+  const double rate = N * K * wb + M * K * 2 > kPgSmallBytes ? 15e6 : 22e6;
+  double best = 0;
+  for (int i = 0; i < kPgShapeCount; ++i) {
+    const PgShape s = kPgShapes[i];
+    const int64_t tiles = ((M + s.bm() - 1) / s.bm()) * ((N + s.bn() - 1) / s.bn());
+    if (tiles > INT32_MAX / 8 || (tune(kTunePg) > 0 && tune(kTunePg) != i + 1)) continue;
+    const int per = s.threads() == 512 ? 1 : 2;  // workgroups of a CU
+    const int64_t slots = (int64_t)device_cus() * per;
+    const double mfma = s.na * s.mb * 2 * 16.0 * (s.threads() / 256) / 2100;  // us a stage
+    for (int S = 1; S <= 8; ++S) {
+      if (S > 1 && (per == 1 || tiles * S > slots || steps / S < 4 || tiles > kCounterSlots)) break;
+      if (tune(kTunePgSplits) > 0 && per == 2 && S != tune(kTunePgSplits)) continue;
+      const int64_t kper = (steps + S - 1) / S;
+      if ((steps + kper - 1) / kper != S) continue;
+      const int64_t rounds = (tiles * S + slots - 1) / slots;
+      const bool two = per == 2 && tiles * S > device_cus();  // both places of a CU taken
+      const double alone = mfma + (wb == 1 ? 0.16 : 0.1);
+      const double chain = (double)(rounds * kper) * (two ? std::max(1.4 * alone, 2 * mfma) : alone);
+      const double copies = (double)(tiles * steps) * pg_stage_bytes(s, wb) / rate;
+      const double cost = std::max(chain, copies) +
+                          (S > 1 ? 5 + (double)tiles * S * s.bm() * s.bn() * 8 / 10e6 : 0);
+      if (!p.ok || cost < best) {
+        best = cost;
+        p.shape = i;
+        p.S = S;
+        p.kper = (int)kper;
+        p.tiles = (int)tiles;
+        p.ok = true;
+      }
+    }
+  }
+  if (!p.ok) return p;
+  size_t off = kCounterBytes;
+  p.rs_off = off;
+  off += align_up((size_t)M * 4, 256);
+  if (gam) {
+    p.xg_off = off;
+    off += align_up((size_t)M * K * 2, 256);
+  }
+  if (p.S > 1) {
+    p.part_off = off;
+    off += align_up((size_t)p.tiles * p.S * kPgShapes[p.shape].bm() * kPgShapes[p.shape].bn() * 4, 256);
+  }
+  p.total = off;
+  return p;
+}
+
+// The plan depends on the sizes, types and tuning keys alone; a thread keeps
+// its last few (the search over shapes and splits is a few us of host time,
+// and a call asks for its plan twice: workspace size and launch).
+PlanPg make_plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
+  struct Entry {
+    int64_t M = -1, N = 0, K = 0;
+    int ct = 0, wt = 0, cus = 0;
+    bool gam = false;
+    unsigned epoch = 0;
+    PlanPg plan;
+  };
+  if (M <= 64) return PlanPg{};
+  constexpr int kEntries = 16;
+  static thread_local Entry cache[kEntries];
+  const unsigned epoch = tune_epoch();
+  const int cus = device_cus();
+  Entry &e = cache[(unsigned)(M * 31 + N * 7 + K + gam + wt) % kEntries];
+  if (e.M != M || e.N != N || e.K != K || e.ct != ct || e.wt != wt || e.gam != gam ||
+      e.cus != cus || e.epoch != epoch) {
+    e.plan = plan_pg(ct, wt, M, N, K, gam);
+    e.M = M;
+    e.N = N;
+    e.K = K;
+    e.ct = ct;
+    e.wt = wt;
+    e.gam = gam;
+    e.cus = cus;
+    e.epoch = epoch;
+  }
+  return e.plan;
+}
+
+int launch_pg(const PlanPg &p, const void *x, const float *gamma, float eps, int norm, PgArgs &a,
+              void *ws, hipStream_t st) {
+  PgKernel k = pg_pick(p.ct, p.wt, p.shape, p.S > 1);
+  if (!k) return MTP_ERR_DTYPE;
+  unsigned char *w8 = (unsigned char *)ws;
+  a.x = x;
+  if (norm || p.gam) {
+    PgPrepKernel pk = pg_prep_pick(p.ct, p.gam);
+    if (!pk) return MTP_ERR_DTYPE;
+    PgPrepArgs pa{};
+    pa.x = x;
+    pa.gamma = gamma;
+    pa.xg = p.gam ? w8 + p.xg_off : nullptr;
+    pa.rs = (float *)(w8 + p.rs_off);
+    pa.K = a.K;
+    pa.norm = norm;
+    pa.eps = eps;
+    hipLaunchKernelGGL(pk, dim3((unsigned)a.M), dim3(256), 0, st, pa);
+    const int s = launch_status();
+    if (s != MTP_OK) return s;
+    a.rs = pa.rs;
+    if (p.gam) a.x = pa.xg;
+  }
+  const PgShape sh = kPgShapes[p.shape];
+  const int wb = dtype_bytes(p.wt);
+  const int lds = pg_stages(sh, wb) * pg_stage_bytes(sh, wb);
+  a.gm = (a.M + sh.bm() - 1) / sh.bm();
+  a.tiles = p.tiles;
+  a.S = p.S;
+  a.kper = p.kper;
+  if (p.S > 1) {
+    a.part = (float *)(w8 + p.part_off);
+    a.ticket = (unsigned *)w8;
+  }
+  const hipError_t e =
+      hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) {
+    note_hip_error(e);
+    return MTP_ERR_LAUNCH;
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)(p.tiles * p.S)), dim3((unsigned)sh.threads()), (size_t)lds, st, a);
+  return launch_status();
+}
+
 int launch_generic_linear(const void *x, int xt, const void *w, int wt, const float *wscale,
                           const void *i4scale, int i4dt, int group, int nib, const void *gamma,
                           int gt, const void *bias, int bt, void *y, int64_t M, int64_t N,
@@ -893,6 +1064,23 @@ int rmsnorm_linear_impl(const void *x, int xt, int64_t M, int64_t K, const void 
     sa.eps = eps;
     sa.scale = scale;
     return launch_sf32(sa, st);
+  }
+  if (M > 64 && aligned && (!gamma || gt == MTP_F32)) {
+    const PlanPg pp = make_plan_pg(xt, wt, M, N, K, gamma != nullptr);
+    if (pp.ok) {
+      if (!ws || ws_bytes < pp.total) return MTP_ERR_WORKSPACE;
+      PgArgs pa{};
+      pa.w = w;
+      pa.wscale = wscale;
+      pa.bias = bias;
+      pa.bias_dt = bt;
+      pa.y = y;
+      pa.M = (int)M;
+      pa.N = (int)N;
+      pa.K = (int)K;
+      pa.scale = scale;
+      return launch_pg(pp, x, (const float *)gamma, eps, norm, pa, ws, st);
+    }
   }
   const int skpm = skp_mode();
   if (skpm != 0 && aligned && (!gamma || gt == MTP_F32)) {
@@ -1371,6 +1559,7 @@ int mtp_set_tuning(const char *name, int64_t value) {
     if (std::strcmp(name, kTuneNames[k]) == 0) {
       if (value < -1 || value > INT32_MAX) return MTP_ERR_ARG;
       g_tune[k].store((int)value, std::memory_order_relaxed);
+      g_tune_epoch.fetch_add(1, std::memory_order_release);
       return MTP_OK;
     }
   }
@@ -1397,6 +1586,8 @@ size_t mtp_rmsnorm_linear_workspace_bytes(int x_dtype, int w_kind, int64_t M, in
   for (int gam = 0; gam < 2; ++gam) {
     PlanX p = make_plan_x(x_dtype, w_kind, M, N, K, gam != 0);
     if (p.ok && p.total > most) most = p.total;
+    PlanPg pg = make_plan_pg(x_dtype, w_kind, M, N, K, gam != 0);
+    if (pg.ok && pg.total > most) most = pg.total;
     PlanSk q = make_plan_sk(x_dtype, w_kind, M, N, K, gam != 0);
     if (q.ok && q.total > most) most = q.total;
     PlanSk qw = make_plan_sk(x_dtype, w_kind, M, N, K, gam != 0, true);

@@ -1,0 +1,89 @@
+"""Prompt GEMM (more than 64 rows) against the oracle, every tile shape and
+K-split forced at the sizes where it can go wrong: rows and columns one past
+a tile, a tile of one row or column, fewer stages than buffers, odd and
+unaligned output rows, splits with an uneven last share. Bound |y - ref| <=
+2e-2 (|ref| + RMS(ref)): x * gamma and y are each rounded once to 8 (bf16)
+or 11 (f16) bits, the sums are fp32."""
+import pytest
+import torch
+
+from conftest import close
+from oracle import eager as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+TYPES = [(torch.bfloat16, "same"), (torch.bfloat16, "fp8"), (torch.float16, "same"),
+         (torch.float16, "fp8")]
+SHAPES = 14  # tile shapes of the kernel
+
+
+def _case(M, N, K, dtype, w, gamma=True, bias=True, norm=True, seed=0):
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(seed + M + 3 * N + 7 * K)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    W = 0.02 * torch.randn(N, K, generator=g)
+    gm = 1 + 0.1 * torch.randn(K, generator=g) if gamma else None
+    b = (0.1 * torch.randn(N, generator=g)).to(dtype) if bias else None
+    dev = [t.to(DEV) if t is not None else None for t in (x, b, gm)]
+    if w == "fp8":
+        wq, ws = O.quantize_fp8_per_channel(W)
+        y = mk.fused_rmsnorm_linear_fp8(dev[0], wq.to(DEV), ws.to(DEV), dev[1], 1e-6,
+                                        gamma=dev[2], norm=norm)
+        ref = O.rmsnorm_linear_fp8(x, wq, ws, b, 1e-6, gamma=gm, norm=norm)
+    else:
+        W = W.to(dtype)
+        y = mk.fused_rmsnorm_linear(dev[0], W.to(DEV), dev[1], 1e-6, gamma=dev[2], norm=norm)
+        ref = O.rmsnorm_linear(x, W, b, 1e-6, 1.0, gamma=gm, norm=norm)
+    assert y.dtype == dtype and y.shape == (M, N)
+    ok, worst = close(y, ref, 2e-2)
+    assert ok, f"worst err/bound = {worst:.3g}"
+    return y
+
+
+@pytest.mark.parametrize("dtype,w", TYPES)
+@pytest.mark.parametrize("shape", range(1, SHAPES + 1))
+def test_every_tile_shape(shape, dtype, w, tune):
+    tune(pg=shape)
+    for M, N, K in ((65, 1, 64), (257, 257, 128), (193, 451, 192), (300, 520, 448)):
+        print(f"case pg shape={shape} {dtype} {w} M={M} N={N} K={K}", flush=True)
+        _case(M, N, K, dtype, w)
+
+
+@pytest.mark.parametrize("dtype,w", TYPES)
+@pytest.mark.parametrize("shape", range(10, SHAPES + 1))
+def test_k_splits(shape, dtype, w, tune):
+    for S in (2, 3, 8):
+        tune(pg=shape, pg_splits=S)
+        for M, N, K in ((65, 70, 64 * 4 * S), (130, 300, 64 * (4 * S + 3))):
+            print(f"case pg split shape={shape} S={S} {dtype} {w} M={M} N={N} K={K}", flush=True)
+            a = _case(M, N, K, dtype, w)
+            assert torch.equal(a, _case(M, N, K, dtype, w))  # fixed order of the sums
+
+
+@pytest.mark.parametrize("gamma,bias,norm", [(False, False, True), (False, True, False),
+                                             (True, False, False)])
+@pytest.mark.parametrize("dtype,w", TYPES)
+@pytest.mark.parametrize("M,N,K", [(65, 513, 1024), (517, 2049, 512), (1000, 96, 2112)])
+def test_planned(M, N, K, dtype, w, gamma, bias, norm):
+    print(f"case pg {dtype} {w} M={M} N={N} K={K} {gamma} {bias} {norm}", flush=True)
+    _case(M, N, K, dtype, w, gamma, bias, norm)
+
+
+def test_graph_replay():
+    """Prep, splits and arrival counts replay; eager calls in between."""
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(9)
+    W = (0.02 * torch.randn(300, 2048, generator=g)).to(torch.bfloat16).to(DEV)
+    x = torch.randn(70, 2048, generator=g).to(torch.bfloat16).to(DEV)
+    gm = (1 + 0.1 * torch.randn(2048, generator=g)).to(DEV)
+    mk.fused_rmsnorm_linear(x, W, gamma=gm)
+    torch.cuda.synchronize()
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr):
+        y = mk.fused_rmsnorm_linear(x, W, gamma=gm)
+    for i in range(4):
+        x.copy_(torch.randn(70, 2048, generator=g).to(torch.bfloat16))
+        ref = mk.fused_rmsnorm_linear(x, W, gamma=gm)
+        gr.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref)
