@@ -66,6 +66,7 @@ enum TuneKey {
   kTuneAttnDec,          // MTP_ATTN_DEC: decode attention kernel, 0 off (MFMA / fallback kernels)
   kTunePg,               // MTP_PG: prompt GEMM, 0 off, n > 0 forces tile shape n - 1
   kTunePgSplits,         // MTP_PG_SPLITS: K-splits of its 4-wave shapes
+  kTuneInt4s,            // MTP_INT4S: skinny INT4 kernel (at most 16 rows), 0 off
   kTuneCount
 };
 int tune(TuneKey k);

@@ -13,6 +13,7 @@
 #include "attn_args.hpp"
 #include "generic.hpp"
 #include "int4g_args.hpp"
+#include "int4s_args.hpp"
 #include "pg_args.hpp"
 #include "quant.hpp"
 #include "sf32_args.hpp"
@@ -33,7 +34,7 @@ std::once_flag g_tune_once;
 const char *const kTuneNames[kTuneCount] = {
     "skl", "sk_splits", "ws_variant", "ws_splits", "skl_waves", "skl_splits",
     "attn_chunk_blocks", "int4_waves", "verify_wstream", "skp", "skp_splits", "skp_ta", "sf32", "skp_h8", "attn32", "sk_xraw",
-    "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw", "attn_dec", "pg", "pg_splits"};
+    "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw", "attn_dec", "pg", "pg_splits", "int4s"};
 
 int env_int(const char *name, int dflt) {
   const char *e = std::getenv(name);
@@ -73,6 +74,7 @@ void tune_init() {
   g_tune[kTuneSklTw].store(env_int("MTP_SKL_TW", -1), std::memory_order_relaxed);
   g_tune[kTuneSkvR8].store(env_int("MTP_SKV_R8", -1), std::memory_order_relaxed);
   g_tune[kTuneSkvTw].store(env_int("MTP_SKV_TW", -1), std::memory_order_relaxed);
+  g_tune[kTuneInt4s].store(env_int("MTP_INT4S", -1), std::memory_order_relaxed);
   g_tune[kTunePgSplits].store(env_int("MTP_PG_SPLITS", -1), std::memory_order_relaxed);
   g_tune[kTunePg].store(env_int("MTP_PG", -1), std::memory_order_relaxed);
   g_tune[kTuneAttnDec].store(env_int("MTP_ATTN_DEC", -1), std::memory_order_relaxed);
@@ -1481,6 +1483,64 @@ bool int4_fast(int64_t M, int64_t N, int64_t K, int64_t group) {
   return ng * int4_ldst(M, N) * 2 < ((int64_t)1 << 31);
 }
 
+// At most 16 rows of 16-bit x, fp16 or fp32 scales, fp32 or no gamma, groups
+// of 32, 64 or whole units of 128 k: one launch of the skinny kernel
+// (int4s.hpp). Returns false where it does not apply.
+bool launch_int4s(const void *x, int xdt, int64_t M, int64_t K, const uint8_t *packed,
+                  const void *scales, int sdt, int64_t N, int64_t group, int nibble,
+                  const void *gamma, int gdt, float eps, int norm, void *y, hipStream_t st,
+                  int *status) {
+  if (tune(kTuneInt4s) == 0 || tune(kTuneInt4Waves) > 0) return false;
+  if (M > kI4sMaxRows || K % 128 != 0) return false;
+  if (gamma && (gdt != MTP_F32 || K > kI4sGammaK)) return false;
+  if (M * K * 2 >= (int64_t)1 << 31) return false;
+  const int64_t ng = (K + group - 1) / group, sb = dtype_bytes(sdt), U = K / 128;
+  // buffer descriptors: a workgroup's rows of W and scales
+  if (256 * (K / 2) >= (int64_t)1 << 31 || 256 * ng * sb >= (int64_t)1 << 31) return false;
+  const int mh = M <= 8 ? 1 : 2;
+  // the scales of a unit in whole aligned pieces when they divide the row
+  const int64_t cg = std::max<int64_t>(1, 128 / group), cb = cg * sb;
+  const bool svec = group <= 128 && ng % cg == 0 &&
+                    ((uintptr_t)scales % (size_t)std::min<int64_t>(cb, 16)) == 0;
+  I4sKernel k = int4s_pick(xdt, gamma != nullptr, sdt, (int)group, mh, svec,
+                           nibble == MTP_NIBBLE_TWOS);
+  if (!k) return false;
+  const int64_t tiles = (N + 7) / 8;
+  I4sArgs a{};
+  a.x = x;
+  a.gamma = (const float *)gamma;
+  a.packed = packed;
+  a.scales = scales;
+  a.y = y;
+  a.M = (int)M;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.group = (int)group;
+  a.ng = (int)ng;
+  a.norm = norm;
+  a.eps = eps;
+  // LDS: the waves' sums of every tile, gamma
+  // one wave per chunk of 256 k at most (enough threads to stage gamma, too)
+  const int nw = (int)std::min<int64_t>(i4s_max_waves(mh), (U + 1) / 2);
+  const int64_t gb = gamma ? K * 4 : 0, tb = (int64_t)nw * i4s_tile_bytes(mh);
+  const int64_t fit = ((int64_t)156 * 1024 - gb) / tb;
+  if (fit < 1) return false;
+  a.nt = (int)std::min<int64_t>({kI4sMaxTiles, fit, (tiles + device_cus() - 1) / device_cus()});
+  const int64_t grid = (tiles + a.nt - 1) / a.nt;
+  const int lds = (int)(tb * a.nt + gb);
+  if (grid > INT32_MAX) return false;
+  const hipError_t e =
+      hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) {
+    note_hip_error(e);
+    *status = MTP_ERR_LAUNCH;
+    return true;
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3((unsigned)(64 * nw)), (size_t)lds, st, a);
+  *status = launch_status();
+  return true;
+}
+
 int launch_int4(const void *x, int xdt, int64_t M, int64_t K, const uint8_t *packed,
                 const void *scales, int sdt, int64_t N, int64_t group, int nibble,
                 const void *gamma, int gdt, float eps, int norm, void *y, void *ws,
@@ -1488,6 +1548,10 @@ int launch_int4(const void *x, int xdt, int64_t M, int64_t K, const uint8_t *pac
   const int64_t ng = (K + group - 1) / group;
   if (!ws || ws_bytes < int4_ws_bytes(M, N, K, ng)) return MTP_ERR_WORKSPACE;
   if (((uintptr_t)ws & 15u) != 0) return MTP_ERR_ALIGN;
+  int status = MTP_OK;
+  if (launch_int4s(x, xdt, M, K, packed, scales, sdt, N, group, nibble, gamma, gdt, eps, norm, y,
+                   st, &status))
+    return status;
   const Int4Tiles tl = int4_tiles(M);
   const int nw = tl.layout == kI4Rows4KHalves ? 8 : 4;
   I4Kernel gemm = int4_gemm_pick(tl.mt, tl.na, tl.layout, nibble == MTP_NIBBLE_TWOS);

@@ -1,0 +1,96 @@
+"""Skinny INT4 kernel (at most 16 rows of 16-bit x) against the oracle, where
+it can go wrong: one and two row halves, columns that end inside a tile and
+inside a workgroup's tiles, K of one unit, odd units, fewer chunks than waves
+and several per wave, every group the lane layout distinguishes, scales whose
+rows are whole pieces and not, both nibble codes. Bound |y - ref| <= rtol
+(|ref| + RMS(ref)): bf16 y 2e-2 (8 bits), f16 5e-3 (x * gamma rounded to 11
+bits, 2^-12 of each term, and y to 11 bits; the sums are fp32)."""
+import pytest
+import torch
+
+from conftest import close
+from oracle import eager as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+RTOL = {torch.bfloat16: 2e-2, torch.float16: 5e-3}
+
+
+def _case(M, N, K, group, dtype, sdt, nibble="ref", gamma=True, norm=True, scale_by=1.0):
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(M + 3 * N + K + group)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    packed = torch.randint(0, 256, (N, K // 2), generator=g).to(torch.uint8)
+    ng = -(-K // group)
+    sc = (scale_by * (0.005 + 0.01 * torch.rand(N, ng, generator=g))).to(sdt)
+    gm = 1 + 0.1 * torch.randn(K, generator=g) if gamma else None
+    print(f"case int4s {dtype} {sdt} M={M} N={N} K={K} group={group} {nibble} {gamma} {norm}",
+          flush=True)
+    y = mk.fused_int4_matmul(x.to(DEV), packed.to(DEV), sc.to(DEV), K, group, nibble=nibble,
+                             gamma=gm.to(DEV) if gamma else None, norm=norm)
+    ref = O.int4_matmul(x, packed, sc, K, group, nibble=nibble, gamma=gm, norm=norm)
+    assert y.shape == (M, N) and y.dtype == dtype
+    ok, worst = close(y, ref, RTOL[dtype])
+    assert ok, f"worst err/bound = {worst:.3g}"
+    return y
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sdt", [torch.float16, torch.float32])
+@pytest.mark.parametrize("group", [32, 64, 128, 256])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 128), (8, 9, 384), (9, 65, 256), (16, 2100, 1152),
+                                   (5, 4111, 4096), (13, 100, 8192), (7, 300, 8320)])
+def test_sizes(M, N, K, group, dtype, sdt):
+    _case(M, N, K, group, dtype, sdt, gamma=K <= 4096)
+
+
+@pytest.mark.parametrize("nibble", ["ref", "twos"])
+@pytest.mark.parametrize("gamma,norm", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("M", [8, 16])
+def test_options(M, gamma, norm, nibble):
+    for sdt in (torch.float16, torch.float32):
+        _case(M, 777, 1280, 64, torch.bfloat16, sdt, nibble, gamma, norm)
+
+
+@pytest.mark.parametrize("M", [3, 12])
+def test_matches_the_tiled_kernel(M, tune):
+    """Same call on the kernel of more rows, and the same bits on a repeat."""
+    a = _case(M, 600, 2048, 128, torch.float16, torch.float16)
+    assert torch.equal(a, _case(M, 600, 2048, 128, torch.float16, torch.float16))
+    tune(int4s=0)
+    b = _case(M, 600, 2048, 128, torch.float16, torch.float16)
+    ok, worst = close(a, b.float().cpu(), 5e-3)
+    assert ok, f"worst err/bound = {worst:.3g}"
+
+
+def test_large_rows_and_small_scales():
+    """Rows far above fp16's range are scaled per unit; scales are not rounded."""
+    import mtp_kernels as mk
+    _case(4, 200, 512, 32, torch.bfloat16, torch.float32, norm=False, scale_by=1e-12)
+    g = torch.Generator().manual_seed(0)
+    x = torch.randn(4, 512, generator=g)
+    x[0] *= 1e30
+    x[1, :128] *= 1e8
+    x[2] *= 1e-30
+    x = x.to(torch.bfloat16)
+    packed = torch.randint(0, 256, (50, 256), generator=g).to(torch.uint8)
+    sc = 0.01 * torch.rand(50, 4, generator=g)
+    y = mk.fused_int4_matmul(x.to(DEV), packed.to(DEV), sc.to(DEV), 512, 128)
+    ref = O.int4_matmul(x, packed, sc, 512, 128)
+    for r in range(4):  # each row against its own scale
+        ok, worst = close(y[r], ref[r], 2e-2)
+        assert ok, f"row {r}: worst err/bound = {worst:.3g}"
+
+
+def test_non_finite_scales_and_x_stay_in_their_columns_and_rows():
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn(3, 384, generator=g).to(torch.float16)
+    x[1, 5] = float("nan")
+    packed = torch.randint(0, 256, (40, 192), generator=g).to(torch.uint8)
+    sc = 0.01 + 0.01 * torch.rand(40, 3, generator=g)
+    sc[7, 2] = float("inf")
+    sc[8, 0] = float("nan")
+    y = mk.fused_int4_matmul(x.to(DEV), packed.to(DEV), sc.to(DEV), 384, 128).cpu()
+    ref = O.int4_matmul(x, packed, sc, 384, 128)
+    assert torch.equal(torch.isfinite(y), torch.isfinite(ref))
