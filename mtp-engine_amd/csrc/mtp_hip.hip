@@ -1712,15 +1712,21 @@ int mtp_fused_int4_matmul(const void *x, int x_dtype, int64_t M, int64_t K, cons
 static int verify_rows_per_chunk(int64_t seq) { return (int)((64 / seq) * seq); }
 
 // Persistent streaming verify (skv.hpp): hidden and W of one dtype (BF16,
-// F16, F32), any bias; 128 bytes of a W row per stage, so K * element bytes
-// a multiple of 512 (the stages of a tile are whole rounds of the 4-slot
-// register ring: K % 256 for 16-bit, K % 128 for fp32); a 256-row tile of W
-// within the reach of one buffer descriptor (W itself may be any size).
-// MTP_VERIFY_WSTREAM selects the column-group kernel instead.
+// F16, F32), any bias; 128 bytes of a W row per stage, so K * element bytes a
+// multiple of 128, and the stages of a tile padded with zeros to whole rounds
+// of the 4-slot register ring where K * element bytes is no multiple of 512
+// (rows of at least 1 KB: at most 3
+// stages in 12. bf16, us: V 16379 K 576 30.1 column-group, 15.8 here, K 2752
+// 122 and 32; V 100000 K 576 49.7 and 34.5; below, K 448 is 41.3 there); a 256-row
+// tile of W within the reach of one buffer descriptor (W itself may be any
+// size). MTP_VERIFY_WSTREAM selects the column-group kernel instead.
+constexpr int64_t kSkvPadMinRow = 1024;
+bool skv_whole_rounds(int ht, int64_t K) { return K * dtype_bytes(ht) % 512 == 0; }
 bool skv_usable(int ht, int64_t V, int64_t K) {
   if (ht != MTP_BF16 && ht != MTP_F16 && ht != MTP_F32) return false;
   const int64_t row = K * dtype_bytes(ht);
-  if (K <= 0 || V <= 0 || row % 512 != 0) return false;
+  if (K <= 0 || V <= 0 || row % kSkUB != 0) return false;
+  if (!skv_whole_rounds(ht, K) && row < kSkvPadMinRow) return false;
   if ((int64_t)kSkvBN * row >= ((int64_t)1 << 31)) return false;
   return tune(kTuneVerifyWstream) <= 0;
 }
@@ -1751,6 +1757,12 @@ static int launch_skv(const void *hidden, int ht, int64_t rows, int64_t K, const
     if (tw < 8) return MTP_ERR_ARG;
   } else if (V >= (int64_t)device_cus() * 64) {
     tw = round_width(V, 1, kSkvBN);
+  } else {
+    // fewer columns leave CUs idle at any width; the stages of a tile are then
+    // a chain of load latencies, shorter with half the loads per stage (bf16,
+    // us: V 16379 K 2752 40.0 at 256 columns, 32.3 at 128, 34.0 at 64, 58 at
+    // 32; V 8000 K 4096 57.0, 48.7, 49.0, 51.7; V 3000 K 4096 46.3, 41.6)
+    tw = kSkvBN / 2;
   }
   const int64_t ntiles = (V + tw - 1) / tw;
   if (ntiles > INT32_MAX) return MTP_ERR_SHAPE;
@@ -1774,7 +1786,8 @@ static int launch_skv(const void *hidden, int ht, int64_t rows, int64_t K, const
     a.K = (int)K;
     a.ntiles = (int)ntiles;
     a.tw = tw;
-    a.nst = (int)(K * dtype_bytes(ht) / kSkUB);  // 128-byte stages of a W row
+    a.kst = (int)(K * dtype_bytes(ht) / kSkUB);  // 128-byte stages of a W row
+    a.nst = (a.kst + 3) / 4 * 4;
     a.keys = (unsigned long long *)(w8 + kSkvKeysOff);
     a.ticket = (unsigned *)w8;
     a.multi = o.multi;
@@ -1865,6 +1878,13 @@ static int verify_common(const void *hidden, int ht, int64_t rows, int64_t K, co
                          WsArgs &a, void *ws, size_t ws_bytes, void *stream) {
   Plan p{};
   const int route = verify_route(hidden, ht, rows, K, w, wt, V, bias, rows_per_chunk, &p);
+  if (route == MTP_VERIFY_ROUTE_STREAM && !skv_whole_rounds(ht, K)) {
+    // these shapes asked for the column-group kernel's workspace before they
+    // streamed, and still do
+    const Plan q = make_plan(ht, wt, rows, V, K, EPI_ARGMAX, rows_per_chunk);
+    if (!q.generic && (!bias || aligned16(bias)) && (!ws || ws_bytes < q.total))
+      return MTP_ERR_WORKSPACE;
+  }
   if (route == MTP_VERIFY_ROUTE_STREAM)
     return launch_skv(hidden, ht, rows, K, w, V, bias, bt, rows_per_chunk, a, ws, ws_bytes,
                       (hipStream_t)stream);

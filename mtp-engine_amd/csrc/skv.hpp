@@ -14,7 +14,8 @@
 // back to back; the stages (128 bytes of every W row of a tile: 64 k of
 // 16-bit W, 32 k of fp32 W) of all its tiles form one sequence, so the
 // register rings run across tile boundaries without draining; each tile's
-// stages start at 7 b mod nst. W is addressed through one buffer descriptor
+// stages (padded with zeros to a multiple of the ring) start at 7 b mod nst.
+// W is addressed through one buffer descriptor
 // per tile (a tile is 256 rows), so W may be any size. 8 waves; wave w owns
 // columns 32 w .. + 31 of every tile against all (<= 64) rows, over every k,
 // so a tile ends with no reduction between waves. Per stage:
@@ -105,9 +106,10 @@ skv_kernel(const SkvArgs a) {
   // W of tile t: rows t * tw .. t * tw + tw - 1 (rows past them, or past N,
   // read zeros)
   const int tw = a.tw;
-  auto w_rsrc = [&](int tile) __attribute__((always_inline)) {
+  auto w_rsrc = [&](int tile, bool on) __attribute__((always_inline)) {
     const int rows = min(tw, N - tile * tw);
-    return make_rsrc((const unsigned char *)a.w + (size_t)tile * tw * ldw, (uint32_t)rows * ldw);
+    return make_rsrc((const unsigned char *)a.w + (size_t)tile * tw * ldw,
+                     on ? (uint32_t)rows * ldw : 0u);
   };
   // W load c (c = wave + 8 i): rows 8 c .. 8 c + 7 of the tile, lane l: row
   // 8 c + l / 8, 16-byte chunk (l % 8) ^ sk_swz(row) of the stage's 128 bytes
@@ -123,7 +125,6 @@ skv_kernel(const SkvArgs a) {
   // stage. 16-bit: k 8 c .. + 7, lane 32 (c % 2) + row % 32 of B-operand
   // block (row / 32, c / 2); fp32: row-major like W.
   const bool xloader = wave < XST / 1024;
-  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.x, (uint32_t)a.M * ldw);
   const int xrow = 8 * wave + (lane >> 3), xc = lane & 7;
   const uint32_t xvo = (uint32_t)xrow * ldw + 16u * (uint32_t)xc;
   const int xlds =
@@ -139,13 +140,16 @@ skv_kernel(const SkvArgs a) {
   auto issue = [&](auto vc, auto slotc) __attribute__((always_inline)) {
     constexpr int v = decltype(vc)::value, slot = decltype(slotc)::value;
     const int str = is_st + rot < nst ? is_st + rot : is_st + rot - nst;
+    const bool on = str < a.kst;  // the padding of a tile to whole ring rounds reads zeros
     if constexpr (v < NWC) {
       const uint32_t off = wvo[v] + (uint32_t)str * (uint32_t)kSkUB;
       wr[slot][v] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc(b + is_i * grid), off, 0, 2));
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc(b + is_i * grid, on), off, 0, 2));
     } else {
       const uint32_t off = xvo + (uint32_t)str * (uint32_t)kSkUB;
-      xr[slot] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
+      xr[slot] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     make_rsrc(a.x, on ? (uint32_t)a.M * ldw : 0u), off, 0, 0));
     }
   };
   auto advance = [&]() __attribute__((always_inline)) {
@@ -373,8 +377,8 @@ skv_kernel(const SkvArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     lds_barrier();
   };
-  // nst is a multiple of NS (the host checks it), so ring slot s % NS of
-  // stage s is the same compile-time slot in every tile
+  // nst is a multiple of NS (the host pads it with stages of zeros), so ring
+  // slot s % NS of stage s is the same compile-time slot in every tile
   for (int i = 0; i < ntl; ++i) {
     load_bias(b + i * grid);
     for (int s0 = 0; s0 < nst; s0 += NS) {
