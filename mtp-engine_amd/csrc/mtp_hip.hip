@@ -1045,13 +1045,26 @@ int rmsnorm_linear_impl(const void *x, int xt, int64_t M, int64_t K, const void 
   a.eps = eps;
   a.scale = scale;
   a.norm = norm;
-  // fp32 x and W, <= 32 rows: one launch of 16-column workgroups, every load
+  // fp32 x and W, <= 32 rows (64, below): one launch of 16-column workgroups, every load
   // in one round trip or each wave's K-range streamed through LDS
   // (launch_sf32 picks; fp32 K 1024 N 4096 16 rows: the planner's tiled
   // kernel 9.9 us)
-  if (xt == MTP_F32 && wt == MTP_F32 && !wscale && tune(kTuneSf32) != 0 && M <= 32 &&
+  // 33 .. 64 rows take two row chunks of it where the tiled kernel's K-splits
+  // cost more than reading W twice: K up to 1536 (beyond, the longer chains of
+  // a wave round more than the tiled kernel's: 2.2e-7 against 1.8e-7 at K
+  // 4096) and at most two workgroups per CU in all (48 rows, us, tiled / this:
+  // K 1024 N 970 19.6 / 7.5, N 4096 18.8 / 13.8, N 8192 20.9 / 26.7; K 256 N
+  // 4096 14.4 / 8.8, N 8192 14.7 / 15.8)
+  const int64_t sf_blocks = (N + 15) / 16;
+  const bool sf_rows =
+      M <= 32 || (M <= kSf32MaxRows && K <= 1536 && sf_blocks <= device_cus());
+  if (xt == MTP_F32 && wt == MTP_F32 && !wscale && tune(kTuneSf32) != 0 && sf_rows &&
       K >= 16 && K <= kSf32StreamMaxK && K % 16 == 0 && aligned && (!gamma || gt == MTP_F32) &&
       tune(kTuneWsVariant) < 0 && tune(kTuneWsSplits) <= 0) {
+    if (M > 32) {  // these rows asked for the tiled kernel's workspace, and still do
+      const PlanX q = make_plan_x(xt, wt, M, N, K, gamma != nullptr);
+      if (q.ok && q.total > 0 && (!ws || ws_bytes < q.total)) return MTP_ERR_WORKSPACE;
+    }
     Sf32Args sa{};
     sa.x = (const float *)x;
     sa.gamma = (const float *)gamma;
@@ -1069,8 +1082,8 @@ int rmsnorm_linear_impl(const void *x, int xt, int64_t M, int64_t K, const void 
   }
   if (M > 64 && aligned && (!gamma || gt == MTP_F32)) {
     const PlanPg pp = make_plan_pg(xt, wt, M, N, K, gamma != nullptr);
-    if (pp.ok) {
-      if (!ws || ws_bytes < pp.total) return MTP_ERR_WORKSPACE;
+    // a smaller workspace is the row-chunk kernel's to take or refuse
+    if (pp.ok && ws && ws_bytes >= pp.total) {
       PgArgs pa{};
       pa.w = w;
       pa.wscale = wscale;

@@ -6,7 +6,7 @@
 namespace mtp {
 
 int launch_sf32(const Sf32Args &a, hipStream_t st) {
-  if (a.M < 1 || a.M > 32 || a.K < 16 || a.K > kSf32StreamMaxK || a.K % 16 != 0 || a.N < 1)
+  if (a.M < 1 || a.M > kSf32MaxRows || a.K < 16 || a.K > kSf32StreamMaxK || a.K % 16 != 0 || a.N < 1)
     return MTP_ERR_SHAPE;
   const unsigned blocks = (unsigned)((a.N + 15) / 16);
   // The one-round-trip kernel (one 139 KB workgroup per CU) only while its
@@ -18,8 +18,8 @@ int launch_sf32(const Sf32Args &a, hipStream_t st) {
   const bool one_trip = a.M <= 16 && a.K <= kSf32MaxK && a.K > 512 &&
                         (int)blocks <= device_cus();
   if (!one_trip) {
-    // streaming form, one or two 16-row tiles
-    const dim3 grid(blocks), block(64 * kSf32sWaves);
+    // streaming form, one or two 16-row tiles (and chunks of two)
+    const dim3 grid(blocks, (unsigned)((a.M + 31) / 32)), block(64 * kSf32sWaves);
     if (a.M > 16) {
       if (a.gamma)
         hipLaunchKernelGGL((sf32s_kernel<true, kSf32sWaves, 2>), grid, block, 0, st, a);

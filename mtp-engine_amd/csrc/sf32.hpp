@@ -213,7 +213,8 @@ __device__ __forceinline__ void sf32_dma4(__amdgpu_buffer_rsrc_t r, unsigned cha
 // flight), its 16 MT MFMAs run (one W fragment feeds every tile), and its
 // slot is refilled with block b + kSf32Ring; refills past the wave's range
 // use out-of-range offsets (zeros, no memory access) so the count stays
-// fixed. Wave t < MT finishes row tile t.
+// fixed. Wave t < MT finishes row tile t. blockIdx.y takes row chunks of 16 MT
+// (33 .. 64 rows: two, which share W through L2).
 template <bool GAM, int NW, int MT>
 __global__ void __launch_bounds__(64 * NW, 1) sf32s_kernel(const Sf32Args a) {
   constexpr int RD = kSf32Ring;
@@ -232,12 +233,14 @@ __global__ void __launch_bounds__(64 * NW, 1) sf32s_kernel(const Sf32Args a) {
   const int g = lane >> 4, r = lane & 15;
   const int n0 = blockIdx.x * 16;
   const int K = a.K;
+  const int m0 = blockIdx.y * 16 * MT;  // first row of this block's row chunk
+  const int M = min(a.M - m0, 16 * MT);
   const int KW = (K + 64 * NW - 1) / (64 * NW) * 64;  // k per wave
   const int nb = KW / 64;                             // blocks per wave
   const int kw0 = KW * wave;
   const __amdgpu_buffer_rsrc_t wrs =
       make_rsrc(a.w + (int64_t)n0 * K, (uint32_t)(min(16, a.N - n0) * K) * 4u);
-  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.x, (uint32_t)(a.M * K) * 4u);
+  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.x + (int64_t)m0 * K, (uint32_t)(M * K) * 4u);
   const __amdgpu_buffer_rsrc_t grs = make_rsrc(a.gamma, GAM ? (uint32_t)K * 4u : 0u);
   // raw bias of the lane's output columns n0 + 4 g + e, before the ring
   uint32_t braw[4] = {0u, 0u, 0u, 0u};
@@ -351,7 +354,7 @@ __global__ void __launch_bounds__(64 * NW, 1) sf32s_kernel(const Sf32Args a) {
   }
   const float rs = a.norm ? 1.0f / sqrtf(sq / (float)K + a.eps) : 1.0f;
   const int m = 16 * tt + r;
-  if (m >= a.M) return;
+  if (m >= M) return;
   const int n = n0 + 4 * g;
   float o[4];
 #pragma unroll
@@ -362,7 +365,7 @@ __global__ void __launch_bounds__(64 * NW, 1) sf32s_kernel(const Sf32Args a) {
                                               : f16_bits_to_f32(braw[e]);
     o[e] = (a.bias ? t[e] * rs + bi : t[e] * rs) * a.scale;
   }
-  float *yr = a.y + (int64_t)m * a.N;
+  float *yr = a.y + (int64_t)(m0 + m) * a.N;
   if (n + 3 < a.N && (a.N & 3) == 0) {
     *(f32x4 *)(yr + n) = f32x4{o[0], o[1], o[2], o[3]};
   } else {

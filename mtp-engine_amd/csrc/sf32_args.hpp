@@ -31,6 +31,7 @@ constexpr int kSf32Waves = 4;
 // 8 x 2 / 4 x 4: fp32 8 x 4096 x 4096 14.0 / 14.0 / 16.0, 8 x 14336 x 4096
 // 42.8 / 48.0 / 53.9, 16 x 4096 x 2048 8.9 / 9.5 / 9.7; 16 waves x 1 block
 // 16.2 at 8 x 4096 x 4096; a deeper W ring than x ring was slower still).
+constexpr int kSf32MaxRows = 64;
 constexpr int kSf32StreamMaxK = 65536;
 constexpr int kSf32Ring = 1;
 constexpr int kSf32sWaves = 8;
