@@ -67,6 +67,7 @@ enum TuneKey {
   kTunePg,               // MTP_PG: prompt GEMM, 0 off, n > 0 forces tile shape n - 1
   kTunePgSplits,         // MTP_PG_SPLITS: K-splits of its 4-wave shapes
   kTuneInt4s,            // MTP_INT4S: skinny INT4 kernel (at most 16 rows), 0 off
+  kTuneInt4Mt,           // MTP_INT4_MT: 32-row x tiles of the tiled INT4 kernel at most (1, 2, 4)
   kTuneCount
 };
 int tune(TuneKey k);

@@ -34,7 +34,7 @@ std::once_flag g_tune_once;
 const char *const kTuneNames[kTuneCount] = {
     "skl", "sk_splits", "ws_variant", "ws_splits", "skl_waves", "skl_splits",
     "attn_chunk_blocks", "int4_waves", "verify_wstream", "skp", "skp_splits", "skp_ta", "sf32", "skp_h8", "attn32", "sk_xraw",
-    "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw", "attn_dec", "pg", "pg_splits", "int4s"};
+    "skw", "skw_tw", "skp_tw", "skl_tw", "skv_r8", "skv_tw", "attn_dec", "pg", "pg_splits", "int4s", "int4_mt"};
 
 int env_int(const char *name, int dflt) {
   const char *e = std::getenv(name);
@@ -74,6 +74,7 @@ void tune_init() {
   g_tune[kTuneSklTw].store(env_int("MTP_SKL_TW", -1), std::memory_order_relaxed);
   g_tune[kTuneSkvR8].store(env_int("MTP_SKV_R8", -1), std::memory_order_relaxed);
   g_tune[kTuneSkvTw].store(env_int("MTP_SKV_TW", -1), std::memory_order_relaxed);
+  g_tune[kTuneInt4Mt].store(env_int("MTP_INT4_MT", -1), std::memory_order_relaxed);
   g_tune[kTuneInt4s].store(env_int("MTP_INT4S", -1), std::memory_order_relaxed);
   g_tune[kTunePgSplits].store(env_int("MTP_PG_SPLITS", -1), std::memory_order_relaxed);
   g_tune[kTunePg].store(env_int("MTP_PG", -1), std::memory_order_relaxed);
@@ -1470,6 +1471,33 @@ Int4Tiles int4_tiles(int64_t M) {
   t.rows = t.gm * 32 * t.mt;
   return t;
 }
+// Tiles of the launch: smaller ones while half of the CUs have no
+// workgroup, and from 128 rows a step further where that pads fewer rows (us,
+// 32-row tiles per workgroup 4 / 2 / 1: M 71 N 5197 K 1024 27.5 / 14.2 / 12.0,
+// M 100 N 1024 K 8192 86.4 / 49.2 / 44.4, M 128 N 14336 K 4096 51.2 / 31.6 /
+// 33.9, M 90 N 20000 K 2048 30.9 / 31.2 / 21.4, M 256 N 28672 K 8192 129 / 193
+// / 199). Never more padded rows or columns than int4_tiles(), which the
+// workspace is laid out for.
+Int4Tiles int4_launch_tiles(int64_t M, int64_t N) {
+  Int4Tiles t = int4_tiles(M);
+  auto shrink = [&] {
+    t.mt /= 2;
+    t.na = 1;
+    t.layout = kI4Rows4;
+    t.bn = int4_bn(t.na);
+    t.gm = (M + 32 * t.mt - 1) / (32 * t.mt);
+    t.rows = t.gm * 32 * t.mt;
+  };
+  if (tune(kTuneInt4Mt) > 0) {
+    while (t.mt > tune(kTuneInt4Mt)) shrink();
+    return t;
+  }
+  if (tune(kTuneInt4Waves) > 0) return t;
+  const int full = t.mt;
+  while (t.mt > 1 && (N + t.bn - 1) / t.bn * t.gm * 2 <= device_cus()) shrink();
+  if (t.mt == 2 && full == 4 && (M + 31) / 32 * 32 < t.rows) shrink();
+  return t;
+}
 // Row stride of the transposed fp16 scales: the columns the GEMM covers.
 int64_t int4_ldst(int64_t M, int64_t N) {
   const int64_t bn = int4_tiles(M).bn;
@@ -1565,7 +1593,7 @@ int launch_int4(const void *x, int xdt, int64_t M, int64_t K, const uint8_t *pac
   if (launch_int4s(x, xdt, M, K, packed, scales, sdt, N, group, nibble, gamma, gdt, eps, norm, y,
                    st, &status))
     return status;
-  const Int4Tiles tl = int4_tiles(M);
+  const Int4Tiles tl = int4_launch_tiles(M, N);
   const int nw = tl.layout == kI4Rows4KHalves ? 8 : 4;
   I4Kernel gemm = int4_gemm_pick(tl.mt, tl.na, tl.layout, nibble == MTP_NIBBLE_TWOS);
   if (!gemm) return MTP_ERR_DTYPE;

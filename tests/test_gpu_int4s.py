@@ -94,3 +94,24 @@ def test_non_finite_scales_and_x_stay_in_their_columns_and_rows():
     y = mk.fused_int4_matmul(x.to(DEV), packed.to(DEV), sc.to(DEV), 384, 128).cpu()
     ref = O.int4_matmul(x, packed, sc, 384, 128)
     assert torch.equal(torch.isfinite(y), torch.isfinite(ref))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,group", [(17, 130, 256, 32), (40, 257, 384, 64), (71, 300, 512, 128),
+                                         (97, 129, 256, 32), (200, 700, 256, 128),
+                                         (257, 40, 256, 64)])
+def test_smaller_tiles_of_few_workgroups(M, N, K, group, dtype, tune):
+    """The tiled kernel's tile per launch, planned and forced to each size."""
+    for mt in (-1, 1, 2, 4):
+        tune(int4_mt=mt)
+        import mtp_kernels as mk
+        g = torch.Generator().manual_seed(M + N)
+        x = torch.randn(M, K, generator=g).to(dtype)
+        packed = torch.randint(0, 256, (N, K // 2), generator=g).to(torch.uint8)
+        sc = 0.005 + 0.01 * torch.rand(N, -(-K // group), generator=g)
+        gm = 1 + 0.1 * torch.randn(K, generator=g)
+        print(f"case int4 tiles mt={mt} {dtype} M={M} N={N} K={K}", flush=True)
+        y = mk.fused_int4_matmul(x.to(DEV), packed.to(DEV), sc.to(DEV), K, group,
+                                 gamma=gm.to(DEV), norm=True)
+        ok, worst = close(y, O.int4_matmul(x, packed, sc, K, group, gamma=gm, norm=True), 2e-2)
+        assert ok, f"mt={mt}: worst err/bound = {worst:.3g}"
