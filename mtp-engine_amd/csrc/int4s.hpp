@@ -23,12 +23,12 @@
 //     Nibbles become fp16 n - 8 (16 (n - 8) at odd k) exactly; the scale
 //     multiplies the fp32 sum of its group, unrounded (a lane's column is one
 //     row of W, so one scalar per lane).
+//   * The waves' sums of a tile meet in LDS at the end, with the sums of
+//     squares of the rows (rs = rstd), in wave order.
 // Measured, 8 rows, N 28672, K 8192, groups of 128, norm and gamma: 48.4 ->
 // 31.5 us a call (3.9 TB/s) against the prep launch and LDS-staged kernel of
 // more rows; N 14336, K 4096: 24.8 -> 13.9. Vector work (decode, x) is half of
 // the time, and the 2-byte scale loads are as many requests as the weights.
-//   * The waves' sums of a tile meet in LDS at the end, with the sums of
-//     squares of the rows (rs = rstd), in wave order.
 #pragma once
 
 #include "int4s_args.hpp"
