@@ -866,6 +866,8 @@ struct PlanPg {
 // {8, 4} 203, {4, 4} 4-wave 272), 517 x 14336 on {6, 3} 67 ({8, 4} 92),
 // 128 x 1000 x 4096 on 4 splits of {2, 1} 13.0 (no split 16.6, {8, 4} 73).
 constexpr int64_t kPgSmallBytes = (int64_t)80 << 20;
+// a launch has less than 2^32 threads in x; the prep takes 256 a row
+constexpr int64_t kPgMaxRows = (int64_t)UINT32_MAX / 256;
 
 PlanPg plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
   PlanPg p;
@@ -875,6 +877,7 @@ PlanPg plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
   if (ct != MTP_BF16 && ct != MTP_F16) return p;
   if (wt != MTP_FP8E4M3 && wt != ct) return p;
   if (tune(kTunePg) == 0 || M <= 64 || N <= 0 || K <= 0 || K % kPgK != 0) return p;
+  if (M > kPgMaxRows) return p;
   if (tune(kTuneWsVariant) >= 0 || tune(kTuneWsSplits) > 0) return p;  // sweeps of wsp
   // buffer descriptors: a tile's rows of x and of W (256 at most)
   if (256 * K * 2 >= (int64_t)1 << 31) return p;
@@ -886,7 +889,8 @@ PlanPg plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
   for (int i = 0; i < kPgShapeCount; ++i) {
     const PgShape s = kPgShapes[i];
     const int64_t tiles = ((M + s.bm() - 1) / s.bm()) * ((N + s.bn() - 1) / s.bn());
-    if (tiles > INT32_MAX / 8 || (tune(kTunePg) > 0 && tune(kTunePg) != i + 1)) continue;
+    if (tiles * s.threads() > (int64_t)UINT32_MAX) continue;
+    if (tune(kTunePg) > 0 && tune(kTunePg) != i + 1) continue;
     const int per = s.threads() == 512 ? 1 : 2;  // workgroups of a CU
     const int64_t slots = (int64_t)device_cus() * per;
     const double mfma = s.na * s.mb * 2 * 16.0 * (s.threads() / 256) / 2100;  // us a stage
@@ -1083,8 +1087,8 @@ int rmsnorm_linear_impl(const void *x, int xt, int64_t M, int64_t K, const void 
   }
   if (M > 64 && aligned && (!gamma || gt == MTP_F32)) {
     const PlanPg pp = make_plan_pg(xt, wt, M, N, K, gamma != nullptr);
-    // a smaller workspace is the row-chunk kernel's to take or refuse
-    if (pp.ok && ws && ws_bytes >= pp.total) {
+    // a smaller or unaligned workspace is the row-chunk kernel's to take or refuse
+    if (pp.ok && ws && aligned16(ws) && ws_bytes >= pp.total) {
       PgArgs pa{};
       pa.w = w;
       pa.wscale = wscale;
@@ -1289,6 +1293,9 @@ DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64
   if (D != 64 && D != 128 && D != 256) return p;
   const bool mfma = (ct == MTP_BF16 || ct == MTP_F16) && D != 256 && NQ > 1 && NQ <= 64 && !kv_fp8;
   if (mfma || tune(kTuneAttnDec) == 0) return p;
+  // launches of 1024 threads a workgroup end below 2^32 threads in x; keys
+  // past the last one of a step still fit an int
+  if (B * H > (int64_t)UINT32_MAX / 1024 || Lc + Lt > INT32_MAX - (1 << 20)) return p;
   p.fast = true;
   const int64_t units = B * H * NQ;
   const int64_t blocks = (Lc + Lt + kAttnBlock - 1) / kAttnBlock;
@@ -1378,11 +1385,12 @@ int launch_attention(AttnArgs &a, int ct, int64_t D, void *ws, size_t ws_bytes, 
                         (!a.kd || aligned16(a.kd)) && (!a.vd || aligned16(a.vd));
   auto dk = dp.fast && dec_rows ? attn_dec_pick(kt, (int)D, a.Lc > 0) : nullptr;
   if (dk) {
-    const size_t need = std::max(p.total, dp.total);
-    if (need > 0 && (!ws || ws_bytes < need)) {
-      // 16-bit calls need their workspace; the others took none before the
-      // chunks and still run without it, one workgroup per query
-      if (p.fast && !a.kv_fp8) return MTP_ERR_WORKSPACE;
+    // 16-bit calls need the workspace of the MFMA kernel's plan, the others
+    // none; what the decode plan needs beyond it only splits the keys
+    if (p.fast && !a.kv_fp8 && p.total > 0 && (!ws || ws_bytes < p.total))
+      return MTP_ERR_WORKSPACE;
+    if (dp.total > 0 && (!ws || ws_bytes < dp.total)) {
+      // one workgroup per query
       dp.nchunks = 1;
       dp.chunk_blocks = (int)((a.Lc + (int64_t)a.Lt + kAttnBlock - 1) / kAttnBlock);
       dp.waves = dec_max_waves(kt);
@@ -1569,7 +1577,7 @@ bool launch_int4s(const void *x, int xdt, int64_t M, int64_t K, const uint8_t *p
   a.nt = (int)std::min<int64_t>({kI4sMaxTiles, fit, (tiles + device_cus() - 1) / device_cus()});
   const int64_t grid = (tiles + a.nt - 1) / a.nt;
   const int lds = (int)(tb * a.nt + gb);
-  if (grid > INT32_MAX) return false;
+  if (grid * 64 * nw > (int64_t)UINT32_MAX) return false;  // threads of a launch in x
   const hipError_t e =
       hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) {

@@ -163,3 +163,25 @@ def test_fp8_entry_without_workspace():
         D ** -0.5, out.data_ptr(), L.stream_handle(q.device))
     assert st == L.OK
     _check(out, ops.causal_attention_fp8(q, k, v, s, s), torch.bfloat16)
+
+
+def test_16bit_needs_no_more_workspace_than_the_mfma_kernel():
+    """A 16-bit call whose MFMA plan has one chunk needs no workspace; where
+    the decode plan would split the keys it then keeps them whole."""
+    from mtp_hip import _lib as L
+    import mtp_kernels as mk
+    B, H, D, N = 24, 12, 64, 512
+    lib = L.load()
+    with L.tuning(attn_dec=0):
+        mfma = lib.mtp_attention_workspace_bytes(L.BF16, B, 1, H, D, 0, N)
+    if mfma:
+        pytest.skip("the MFMA kernel splits these keys on this device")
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(B, H, D, generator=g).to(torch.bfloat16).to(DEV)
+    k, v = (torch.randn(B, H, N, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    out = torch.empty_like(q)
+    st = lib.mtp_fused_causal_attention(q.data_ptr(), L.BF16, B, H, D, k.data_ptr(), v.data_ptr(),
+                                        N, D ** -0.5, out.data_ptr(), None, 0,
+                                        L.stream_handle(q.device))
+    assert st == L.OK
+    _check(out, mk.fused_causal_attention(q, k, v), torch.bfloat16)
