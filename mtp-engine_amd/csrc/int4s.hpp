@@ -25,10 +25,13 @@
 //     row of W, so one scalar per lane).
 //   * The waves' sums of a tile meet in LDS at the end, with the sums of
 //     squares of the rows (rs = rstd), in wave order.
+//   * Scales: one 2-byte load per tile and chunk is as many requests as the
+//     weights take, so the workgroup's scale rows are staged in LDS with
+//     16-byte loads before the first tile where they fit (31.5 -> 30.0 us).
 // Measured, 8 rows, N 28672, K 8192, groups of 128, norm and gamma: 48.4 ->
-// 31.5 us a call (3.9 TB/s) against the prep launch and LDS-staged kernel of
-// more rows; N 14336, K 4096: 24.8 -> 13.9. Vector work (decode, x) is half of
-// the time, and the 2-byte scale loads are as many requests as the weights.
+// 30.0 us a call (4.1 TB/s) against the prep launch and LDS-staged kernel of
+// more rows; N 14336, K 4096: 24.8 -> 13.3. Vector work (decode, x) is half of
+// the time. The ring is a tile shorter with LDS scales (128 registers).
 #pragma once
 
 #include "int4s_args.hpp"
@@ -63,14 +66,15 @@ __device__ __forceinline__ u32x4 i4s_transpose(u32x4 a) {
   return u32x4{lo[0], lo[1], hi[0], hi[1]};
 }
 
-template <int XT, bool GAM, int SDT, int GRP, int MH, bool SVEC, bool TWOS>
+template <int XT, bool GAM, int SDT, int GRP, int MH, int SM, bool TWOS>
 __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4sArgs a) {
   constexpr int SB = SDT == MTP_F32 ? 4 : 2;
   constexpr int NG = 128 / GRP;  // scale groups per unit
+  constexpr bool SVEC = SM == kI4sScaleVec, SLDS = SM == kI4sScaleLds;
   // registers of a unit's scales: whole pieces of the row, or one each
-  constexpr int SR = !SVEC ? NG : NG * SB < 4 ? 1 : NG * SB / 4;
+  constexpr int SR = SLDS ? 1 : !SVEC ? NG : NG * SB < 4 ? 1 : NG * SB / 4;
   // ring: tiles in flight (128 registers up to 8 rows)
-  constexpr int R = MH == 2 ? 8 : SR == 1 ? 7 : SR == 2 ? 5 : 4;
+  constexpr int R = MH == 2 ? 8 : SLDS ? (NG == 4 ? 5 : 6) : SR == 1 ? 7 : SR == 2 ? 5 : 4;
   constexpr int SPG = GRP / 32;  // MFMA k-steps per group
   constexpr int AL = 32 * MH;    // lanes of a tile's sums kept (8 or 16 rows)
   extern __shared__ __attribute__((aligned(16))) f32x4 s_acc[];  // [wave][tile][AL], gamma [K]
@@ -106,6 +110,7 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
     const bool in = c < nchunk && t < ntl;
     const uint32_t wo = (uint32_t)t * 8u * ldw + (uint32_t)c * 128u;
     w[S] = bload16_nt(make_rsrc(wbase + wo, in ? wbytes - wo : 0u), wvo);
+    if constexpr (SLDS) return;
     const uint32_t so = (uint32_t)t * 8u * spitch;
     const __amdgpu_buffer_rsrc_t srs = make_rsrc(sbase + so, in ? sbytes - so : 0u);
     const int un = 2 * c + half;
@@ -158,7 +163,11 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
                        MH == 1 && k_of(c, j) >= K ? kOOB : xvo);
     }
   };
-  const float *const s_gam = (const float *)(s_acc + nw * a.nt * AL);
+  float *const s_gam = (float *)(s_acc + nw * a.nt * AL);
+  // scale rows of the workgroup's columns, 4 bytes apart beyond their length
+  // (the 8 columns of a tile in different banks)
+  unsigned char *const s_scl = (unsigned char *)(s_gam + (GAM ? K : 0));
+  const uint32_t slp = spitch + 4u;
   auto make_x = [&](int c) __attribute__((always_inline)) {
     auto values = [&](int j, float(&v)[8], bool squares) __attribute__((always_inline)) {
 #pragma unroll
@@ -237,8 +246,19 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
   // the first unit's columns, 8 .. 15 for the second's), and their slot
   const bool keep = MH == 2 || (lg >> 1) == half;
   const int aslot = MH == 2 ? lane : l16 + 16 * (lg & 1);
-  auto multiply = [&](auto slot_c, int t, bool first) __attribute__((always_inline)) {
+  auto multiply = [&](auto slot_c, int c, int t, bool first) __attribute__((always_inline)) {
     constexpr int S = decltype(slot_c)::value;
+    float sl[NG];
+    if constexpr (SLDS) {
+      const int un = 2 * c + half;
+      const uint32_t gr = (uint32_t)min(un, U - 1) * 128u / (uint32_t)a.group;
+      const unsigned char *const sp = s_scl + (uint32_t)(t * 8 + row8) * slp + gr * SB;
+#pragma unroll
+      for (int i = 0; i < NG; ++i) {
+        const float v = SB == 4 ? ((const float *)sp)[i] : f16_bits_to_f32(((const uint16_t *)sp)[i]);
+        sl[i] = un < U ? v : 0.f;
+      }
+    }
     const u32x4 d = i4s_transpose(w[S]);
     const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
     f32x4 acc = zero, p = zero, p1 = zero;
@@ -255,7 +275,7 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
       p = mfma16<MTP_F16>(xf[j], b, p);
       if constexpr (MH == 2) p1 = mfma16<MTP_F16>(xf[XJ - 4 + j], b, p1);
       if ((j + 1) % SPG == 0) {
-        const float s = scale_of(slot_c, j / SPG);
+        const float s = SLDS ? sl[j / SPG] : scale_of(slot_c, j / SPG);
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = fmaf(MH == 2 && half ? p1[r] : p[r], s, acc[r]);
         p = zero;
@@ -284,19 +304,37 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
     for (int i = 0; i < GV; ++i)
       gv[i] = __builtin_bit_cast(f32x4, bload16(grs, 16u * (uint32_t)(th + 64 * nw * i)));
   }
+  u32x4 sv[SLDS ? i4s_scale_loads(MH) : 1];
+  if constexpr (SLDS) {
+    const __amdgpu_buffer_rsrc_t srs = make_rsrc(sbase, sbytes);
+#pragma unroll
+    for (int i = 0; i < i4s_scale_loads(MH); ++i) sv[i] = bload16(srs, 16u * (uint32_t)(th + 64 * nw * i));
+  }
   fetch_x(wave);
   __builtin_amdgcn_sched_barrier(0);
   static_for<0, R - 1>([&](auto s) { load(s, wave, decltype(s)::value); });
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (GAM) {  // the oldest loads: nothing behind them is waited for
-    float *const sg = (float *)(s_acc + nw * a.nt * AL);
+  // the oldest loads: nothing behind them is waited for
+  if constexpr (GAM) {
 #pragma unroll
     for (int i = 0; i < GV; ++i) {
       const int k = 4 * (th + 64 * nw * i);
-      if (k < K) *(f32x4 *)(sg + k) = gv[i];
+      if (k < K) *(f32x4 *)(s_gam + k) = gv[i];
     }
-    lds_barrier();
   }
+  if constexpr (SLDS) {
+#pragma unroll
+    for (int i = 0; i < i4s_scale_loads(MH); ++i) {
+      const uint32_t o = 16u * (uint32_t)(th + 64 * nw * i);
+      if (o < sbytes) {  // rows are whole 16-byte pieces
+        const uint32_t row = o / spitch;
+        uint32_t *const q = (uint32_t *)(s_scl + row * slp + (o - row * spitch));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = sv[i][e];
+      }
+    }
+  }
+  if constexpr (GAM || SLDS) lds_barrier();
   for (int c = wave; c < nchunk; c += nw) {
     make_x(c);
     fetch_x(c + nw);  // past the last chunk: zeros
@@ -307,7 +345,7 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
         const int ta = t0 + SL + R - 1;
         load(std::integral_constant<int, (SL + R - 1) % R>{}, ta < ntp ? c : c + nw,
              ta < ntp ? ta : ta - ntp);
-        if (t0 + SL < ntl) multiply(s, t0 + SL, c == wave);
+        if (t0 + SL < ntl) multiply(s, c, t0 + SL, c == wave);
       });
       t0 += R;
     } while (t0 < ntp);

@@ -14,6 +14,12 @@ constexpr int kI4sMaxTiles = 32;  // 8-column tiles per workgroup
 constexpr int i4s_max_waves(int mh) { return mh == 1 ? 16 : 8; }
 constexpr int i4s_tile_bytes(int mh) { return 512 * mh; }
 
+// How scales reach the lanes: one load each, whole pieces of a unit's scales,
+// or the workgroup's scale rows kept in LDS (16-byte loads, this many a thread
+// at most).
+enum { kI4sScaleEach = 0, kI4sScaleVec = 1, kI4sScaleLds = 2 };
+constexpr int i4s_scale_loads(int mh) { return mh; }
+
 struct I4sArgs {
   const void *x;          // [M, K] BF16 / F16
   const float *gamma;     // [K] or null
@@ -28,8 +34,8 @@ struct I4sArgs {
 typedef void (*I4sKernel)(I4sArgs);
 // x dtype (BF16 / F16), gamma present, scale dtype (F16 / F32), group (32,
 // 64, or 128 for every multiple of 128),
-// 8-row halves (1, 2), scales of a unit being whole aligned pieces of their row,
+// 8-row halves (1, 2), how scales are read (kI4sScale*),
 // two's-complement nibbles; or null.
-I4sKernel int4s_pick(int xdt, bool gam, int sdt, int group, int mh, bool svec, bool twos);
+I4sKernel int4s_pick(int xdt, bool gam, int sdt, int group, int mh, int sm, bool twos);
 
 }  // namespace mtp

@@ -1551,9 +1551,6 @@ bool launch_int4s(const void *x, int xdt, int64_t M, int64_t K, const uint8_t *p
   const int64_t cg = std::max<int64_t>(1, 128 / group), cb = cg * sb;
   const bool svec = group <= 128 && ng % cg == 0 &&
                     ((uintptr_t)scales % (size_t)std::min<int64_t>(cb, 16)) == 0;
-  I4sKernel k = int4s_pick(xdt, gamma != nullptr, sdt, (int)group, mh, svec,
-                           nibble == MTP_NIBBLE_TWOS);
-  if (!k) return false;
   const int64_t tiles = (N + 7) / 8;
   I4sArgs a{};
   a.x = x;
@@ -1572,11 +1569,24 @@ bool launch_int4s(const void *x, int xdt, int64_t M, int64_t K, const uint8_t *p
   // one wave per chunk of 256 k at most (enough threads to stage gamma, too)
   const int nw = (int)std::min<int64_t>(i4s_max_waves(mh), (U + 1) / 2);
   const int64_t gb = gamma ? K * 4 : 0, tb = (int64_t)nw * i4s_tile_bytes(mh);
-  const int64_t fit = ((int64_t)156 * 1024 - gb) / tb;
+  constexpr int64_t kLds = 159 * 1024;  // 160 KB less the static arrays
+  const int64_t fit = (kLds - gb) / tb;
   if (fit < 1) return false;
   a.nt = (int)std::min<int64_t>({kI4sMaxTiles, fit, (tiles + device_cus() - 1) / device_cus()});
   const int64_t grid = (tiles + a.nt - 1) / a.nt;
-  const int lds = (int)(tb * a.nt + gb);
+  // Scale rows through LDS where they are whole 16-byte pieces and fit beside
+  // the sums (us, 2-byte loads / LDS: M 8 N 28672 K 8192 G 128 31.5 / 30.0,
+  // M 5 N 4096 K 4096 G 32 11.5 / 11.0, M 12 N 20000 K 2048 G 64 fp32 13.9 /
+  // 12.6, M 2 N 14336 K 4096 G 128 13.7 / 13.3)
+  const int64_t srow = ng * sb, sl = a.nt * 8 * (srow + 4);
+  const bool slds = tune(kTuneInt4s) != 2 && srow % 16 == 0 && aligned16(scales) &&
+                    tb * a.nt + gb + sl <= kLds &&
+                    a.nt * 8 * srow <= (int64_t)i4s_scale_loads(mh) * 64 * nw * 16;
+  const int lds = (int)(tb * a.nt + gb + (slds ? sl : 0));
+  I4sKernel k = int4s_pick(xdt, gamma != nullptr, sdt, (int)group, mh,
+                           slds ? kI4sScaleLds : svec ? kI4sScaleVec : kI4sScaleEach,
+                           nibble == MTP_NIBBLE_TWOS);
+  if (!k) return false;
   if (grid * 64 * nw > (int64_t)UINT32_MAX) return false;  // threads of a launch in x
   const hipError_t e =
       hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);

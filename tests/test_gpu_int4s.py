@@ -115,3 +115,17 @@ def test_smaller_tiles_of_few_workgroups(M, N, K, group, dtype, tune):
                                  gamma=gm.to(DEV), norm=True)
         ok, worst = close(y, O.int4_matmul(x, packed, sc, K, group, gamma=gm, norm=True), 2e-2)
         assert ok, f"mt={mt}: worst err/bound = {worst:.3g}"
+
+
+@pytest.mark.parametrize("M,N,K,group,sdt", [(8, 1029, 1024, 128, torch.float16),
+                                             (3, 20000, 3072, 128, torch.float32),
+                                             (16, 2053, 2560, 32, torch.float16),
+                                             (9, 8, 1024, 256, torch.float32),
+                                             (1, 4099, 8192, 64, torch.float16)])
+def test_scales_through_lds_change_no_bit(M, N, K, group, sdt, tune):
+    """Whole 16-byte scale rows go through LDS: the same sums in the same
+    order as with one load per tile, also where columns end inside a tile, a
+    chunk has one unit and a wave several chunks."""
+    y = _case(M, N, K, group, torch.bfloat16, sdt)
+    tune(int4s=2)
+    assert torch.equal(y, _case(M, N, K, group, torch.bfloat16, sdt))
