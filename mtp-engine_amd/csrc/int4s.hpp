@@ -203,10 +203,10 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
       }
       mx = max_over_lane_groups(mx);  // of the A row, in its four lanes
       int e = 0;
-      if (mx > 0.f && mx <= 3.0e38f) {
+      if (mx > 0.f && mx < INFINITY) {
         int ex;
-        frexpf(mx, &ex);
-        e = min(max(ex - 15, -100), 100);
+        frexpf(mx, &ex);  // at most 128
+        e = max(ex - 15, -100);
       }
       const float mul = ldexpf(1.0f, -e), odd = mul * 0.0625f;
       back[u] = ldexpf(1.0f, e);
@@ -354,10 +354,41 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
   if (lane < 16) s_ss[wave][lane] = ss;
   __syncthreads();
 
+  // One output by its definition, sum over k of (x * f * gamma) * ((nib - 8) *
+  // scale) in fp32, by the whole wave.
+  auto direct = [&](int m, int n, float f) {
+    const int64_t nk = (int64_t)n * ldw;
+    float t = 0.f;
+    for (int k = 8 * lane; k < K; k += 512) {
+      const u32x4 xv = *(const u32x4 *)((const uint16_t *)a.x + (int64_t)m * K + k);
+      const uint32_t wv = *(const uint32_t *)(a.packed + nk + k / 2);
+      const int64_t si = (int64_t)n * a.ng + k / a.group;
+      const float s = SB == 4 ? ((const float *)a.scales)[si]
+                              : f16_bits_to_f32(((const uint16_t *)a.scales)[si]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t nib = (wv >> (4 * i)) & 15u;
+        const f32x2 p = unpack2<XT>(xv[i / 2]);
+        float v = p[i & 1] * f;
+        if constexpr (GAM) v *= s_gam[k + i];
+        t = fmaf(v, (float)((int)(TWOS ? nib ^ 8u : nib) - 8) * s, t);
+      }
+    }
+#pragma unroll
+    for (int w = 1; w < 64; w <<= 1) t += __shfl_xor(t, w, 64);
+    return t;
+  };
+
   // ---- the waves' sums in wave order (first unit's and second unit's
-  // columns), row factor, output: thread (tile, column, rows 4 q .. 4 q + 3)
+  // columns), row factor, output: thread (tile, column, rows 4 q .. 4 q + 3).
+  // The sums hold x * gamma before the row factor, so they can leave fp32's
+  // range where the output does not (a row whose squares overflow has the
+  // factor 0 and is 0; a huge gamma): an output that is not finite, of a row
+  // without NaN, is computed again in the order of the definition.
   constexpr int RQ = 2 * MH;
-  for (int i = th; i < ntl * 8 * RQ; i += 64 * nw) {
+  const int nout = ntl * 8 * RQ;
+  for (int i0 = 64 * wave; i0 < nout; i0 += 64 * nw) {
+    const int i = min(i0 + lane, nout - 1);
     const int t = i / (8 * RQ), rem = i - t * 8 * RQ, q4 = rem >> 3, col = rem & 7;
     const int n = n0 + t * 8 + col;
     const int s0 = col + 16 * q4, s1 = 8 + col + 16 * q4;
@@ -369,14 +400,22 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = 4 * q4 + r;
-      if (m >= a.M || n >= a.N) continue;
+      const bool on = i0 + lane < nout && m < a.M && n < a.N;
       float f = 1.f;
       if (a.norm) {
         float s2 = 0.f;
         for (int q = 0; q < nw; ++q) s2 += MH == 1 ? s_ss[q][m] + s_ss[q][m + 8] : s_ss[q][m];
         f = 1.0f / sqrtf(s2 / (float)K + a.eps);
       }
-      ((uint16_t *)a.y)[(int64_t)m * a.N + n] = (uint16_t)pack2<XT>(v[r] * f, 0.f);
+      float y = v[r] * f;
+      if (a.norm) {
+        for (uint64_t bad = __ballot(on && f == f && !(fabsf(y) < INFINITY)); bad; bad &= bad - 1) {
+          const int l = __builtin_ctzll(bad);
+          const float z = direct(__shfl(m, l, 64), __shfl(n, l, 64), __shfl(f, l, 64));
+          y = lane == l ? z : y;
+        }
+      }
+      if (on) ((uint16_t *)a.y)[(int64_t)m * a.N + n] = (uint16_t)pack2<XT>(y, 0.f);
     }
   }
 }

@@ -129,3 +129,53 @@ def test_scales_through_lds_change_no_bit(M, N, K, group, sdt, tune):
     y = _case(M, N, K, group, torch.bfloat16, sdt)
     tune(int4s=2)
     assert torch.equal(y, _case(M, N, K, group, torch.bfloat16, sdt))
+
+
+@pytest.mark.parametrize("gamma", [None, 1.0, 1e30])
+@pytest.mark.parametrize("M", [6, 13])
+def test_rows_whose_sums_leave_fp32_under_the_norm(M, gamma, tune):
+    """The sums hold x * gamma before the row factor: rows whose squares
+    overflow are 0 (inf in x: NaN) and a huge gamma is finite, as in the
+    oracle (and, but for the huge gamma, in the kernel of more rows)."""
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, 512, generator=g).to(torch.bfloat16)
+    for r, mag in enumerate((1e12, 1e20, 1e35, 1e36)):
+        x[r] *= mag
+    x[4, ::7] = 3.3e38
+    x[5, 3] = float("inf")
+    packed = torch.randint(0, 256, (50, 256), generator=g).to(torch.uint8)
+    sc = 0.01 * torch.rand(50, 4, generator=g)
+    gm = gamma * (1 + 0.1 * torch.randn(512, generator=g)) if gamma else None
+    ref = O.int4_matmul(x, packed, sc, 512, 128, gamma=gm, norm=True)
+    args = [t.to(DEV) for t in (x, packed, sc)]
+    gd = gm.to(DEV) if gamma else None
+    for keys in ({}, {"int4s": 2}, {"int4s": 0}):
+        if keys == {"int4s": 0} and gamma == 1e30:
+            continue
+        tune(**keys)
+        print(f"case int4s large rows M={M} gamma={gamma} {keys}", flush=True)
+        y = mk.fused_int4_matmul(*args, 512, 128, gamma=gd, norm=True).cpu()
+        assert torch.equal(torch.isfinite(y), torch.isfinite(ref))
+        for r in (0, 1, 2, 3, 4, *range(6, M)):
+            ok, worst = close(y[r], ref[r], 2e-2)
+            assert ok, f"{keys} row {r}: worst err/bound = {worst:.3g}"
+
+
+@pytest.mark.parametrize("M", [3, 12])
+def test_large_rows_without_the_norm(M):
+    """A unit's power of two reaches every finite x."""
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, 256, generator=g)
+    x[0] *= 1e35
+    x[1] *= 1e36
+    x[2, :128] *= 1e37
+    x = x.to(torch.bfloat16)
+    packed = torch.randint(0, 256, (50, 128), generator=g).to(torch.uint8)
+    sc = 0.01 * torch.rand(50, 2, generator=g)
+    y = mk.fused_int4_matmul(x.to(DEV), packed.to(DEV), sc.to(DEV), 256, 128).cpu()
+    ref = O.int4_matmul(x, packed, sc, 256, 128)
+    for r in range(M):
+        ok, worst = close(y[r], ref[r], 2e-2)
+        assert ok, f"row {r}: worst err/bound = {worst:.3g}"
