@@ -1385,9 +1385,10 @@ int launch_attention(AttnArgs &a, int ct, int64_t D, void *ws, size_t ws_bytes, 
                         (!a.kd || aligned16(a.kd)) && (!a.vd || aligned16(a.vd));
   auto dk = dp.fast && dec_rows ? attn_dec_pick(kt, (int)D, a.Lc > 0) : nullptr;
   if (dk) {
-    // 16-bit calls need the workspace of the MFMA kernel's plan, the others
-    // none; what the decode plan needs beyond it only splits the keys
-    if (p.fast && !a.kv_fp8 && p.total > 0 && (!ws || ws_bytes < p.total))
+    // calls of the MFMA kernel's forms need the workspace of its plan, the
+    // others (an unaligned q or out among them) none; what the decode plan
+    // needs beyond it only splits the keys
+    if (p.fast && strides8 && aligned && !a.kv_fp8 && p.total > 0 && (!ws || ws_bytes < p.total))
       return MTP_ERR_WORKSPACE;
     if (dp.total > 0 && (!ws || ws_bytes < dp.total)) {
       // one workgroup per query

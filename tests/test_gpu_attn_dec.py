@@ -185,3 +185,32 @@ def test_16bit_needs_no_more_workspace_than_the_mfma_kernel():
                                         L.stream_handle(q.device))
     assert st == L.OK
     _check(out, mk.fused_causal_attention(q, k, v), torch.bfloat16)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("which", ["q", "out"])
+def test_unaligned_query_or_output_needs_no_workspace(which, dtype):
+    """q or out off a 16-byte boundary is none of the MFMA kernel's calls:
+    with no workspace the keys stay in one workgroup, with one they split."""
+    from mtp_hip import _lib as L
+    import mtp_kernels as mk
+    B, H, D, N = 1, 2, 128, 1000
+    lib = L.load()
+    code = L.BF16 if dtype == torch.bfloat16 else L.F16
+    need = lib.mtp_attention_workspace_bytes(code, B, 1, H, D, 0, N)
+    assert need > 0
+    g = torch.Generator().manual_seed(6)
+    k, v = (torch.randn(B, H, N, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+    bufs = [torch.zeros(B * H * D + 1, dtype=dtype, device=DEV) for _ in range(2)]
+    q, out = (b[1:] if name == which else b[:-1] for b, name in zip(bufs, ("q", "out")))
+    q = q.view(B, H, D).copy_(torch.randn(B, H, D, generator=g))
+    ref = O.causal_attention(q.cpu(), k.cpu(), v.cpu())
+    ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
+    for w, n in ((None, 0), (ws.data_ptr(), need)):
+        print(f"case decode unaligned {which} {dtype} workspace={n}", flush=True)
+        st = lib.mtp_fused_causal_attention(q.data_ptr(), code, B, H, D, k.data_ptr(), v.data_ptr(),
+                                            N, D ** -0.5, out.data_ptr(), w, n,
+                                            L.stream_handle(q.device))
+        assert st == L.OK
+        _check(out.view(B, H, D), ref, dtype)
+    _check(mk.fused_causal_attention(q, k, v), ref, dtype)
