@@ -1701,8 +1701,10 @@ int mtp_get_tuning(const char *name, int64_t *value) {
   return MTP_ERR_ARG;
 }
 
-size_t mtp_rmsnorm_linear_workspace_bytes(int x_dtype, int w_kind, int64_t M, int64_t N,
-                                          int64_t K) {
+// Most workspace of any kernel the call may take; without `prompt`, of those
+// that refuse a smaller one (the prompt GEMM leaves such calls to the others).
+static size_t linear_ws_bytes(int x_dtype, int w_kind, int64_t M, int64_t N, int64_t K,
+                              bool prompt) {
   // packed INT4: enough for every group the MFMA path takes (group >= 32)
   if (w_kind == MTP_U8) return int4_fast(M, N, K, 32) ? int4_ws_bytes(M, N, K, K / 32) : 0;
   // enough for the call with or without gamma
@@ -1710,8 +1712,10 @@ size_t mtp_rmsnorm_linear_workspace_bytes(int x_dtype, int w_kind, int64_t M, in
   for (int gam = 0; gam < 2; ++gam) {
     PlanX p = make_plan_x(x_dtype, w_kind, M, N, K, gam != 0);
     if (p.ok && p.total > most) most = p.total;
-    PlanPg pg = make_plan_pg(x_dtype, w_kind, M, N, K, gam != 0);
-    if (pg.ok && pg.total > most) most = pg.total;
+    if (prompt) {
+      PlanPg pg = make_plan_pg(x_dtype, w_kind, M, N, K, gam != 0);
+      if (pg.ok && pg.total > most) most = pg.total;
+    }
     PlanSk q = make_plan_sk(x_dtype, w_kind, M, N, K, gam != 0);
     if (q.ok && q.total > most) most = q.total;
     PlanSk qw = make_plan_sk(x_dtype, w_kind, M, N, K, gam != 0, true);
@@ -1722,6 +1726,11 @@ size_t mtp_rmsnorm_linear_workspace_bytes(int x_dtype, int w_kind, int64_t M, in
     if (q2.ok && q2.total > most) most = q2.total;
   }
   return most;
+}
+
+size_t mtp_rmsnorm_linear_workspace_bytes(int x_dtype, int w_kind, int64_t M, int64_t N,
+                                          int64_t K) {
+  return linear_ws_bytes(x_dtype, w_kind, M, N, K, true);
 }
 
 int mtp_fused_rmsnorm_linear(const void *x, int x_dtype, int64_t M, int64_t K, const void *weight,
@@ -2165,18 +2174,30 @@ int mtp_fused_causal_attention_fp8_ws(const void *q, int dtype, int64_t B, int64
 // Tree monolith: attention over the masked keys into an intermediate
 // [B * H, D] (q's dtype) at the end of the workspace, then RMSNorm over the
 // head dimension (gamma rms_w) and the projection onto proj_w's rows.
-static size_t monolith_tmp_off(int dtype, int64_t B, int64_t H, int64_t D, int64_t L, int w_kind,
-                               int64_t N) {
-  const size_t att = attn_ws_bytes(dtype, B, 1, H, D, 0, L);
-  const size_t lin = mtp_rmsnorm_linear_workspace_bytes(dtype, w_kind, B * H, N, D);
-  return align_up(std::max(kCounterBytes, std::max(att, lin)), 256);
+// What its two stages ask for: `least` is what they cannot run without, `best`
+// what their plans take beyond it (key chunks of the decode kernel, the prompt
+// GEMM's x * gamma), each ahead of the intermediate.
+struct MonolithSpace {
+  size_t least, best, tmp;
+};
+static MonolithSpace monolith_space(int dtype, int64_t B, int64_t H, int64_t D, int64_t L,
+                                    int w_kind, int64_t N) {
+  MonolithSpace m;
+  const size_t att = make_attn_plan(dtype, B, 1, H, D, 0, L).total;
+  const size_t lin = linear_ws_bytes(dtype, w_kind, B * H, N, D, false);
+  m.least = align_up(std::max({kCounterBytes, att, lin}), 256);
+  m.best = align_up(std::max({m.least, make_dec_plan(dtype, B, 1, H, D, 0, L, false).total,
+                              linear_ws_bytes(dtype, w_kind, B * H, N, D, true)}),
+                    256);
+  m.tmp = align_up((size_t)(B * H * D) * dtype_bytes(dtype), 256);
+  return m;
 }
 
 size_t mtp_tree_attn_rmsnorm_linear_workspace_bytes(int dtype, int64_t B, int64_t H, int64_t D,
                                                     int64_t L, int w_kind, int64_t N) {
   if (B <= 0 || H <= 0 || D <= 0 || L < 0 || N <= 0) return 0;
-  return monolith_tmp_off(dtype, B, H, D, L, w_kind, N) +
-         align_up((size_t)(B * H * D) * dtype_bytes(dtype), 256);
+  const MonolithSpace m = monolith_space(dtype, B, H, D, L, w_kind, N);
+  return m.best + m.tmp;
 }
 
 int mtp_fused_tree_attn_rmsnorm_linear(const void *q, int dtype, int64_t B, int64_t H, int64_t D,
@@ -2194,10 +2215,10 @@ int mtp_fused_tree_attn_rmsnorm_linear(const void *q, int dtype, int64_t B, int6
     return MTP_ERR_SHAPE;
   if (B == 0 || H == 0 || N == 0) return MTP_OK;
   if (!q || !out || !proj_w || (L > 0 && (!k || !v || !mask))) return MTP_ERR_NULL;
-  const size_t need = mtp_tree_attn_rmsnorm_linear_workspace_bytes(dtype, B, H, D, L,
-                                                                   wscale ? MTP_FP8E4M3 : w_dtype, N);
-  if (!workspace || workspace_bytes < need) return MTP_ERR_WORKSPACE;
-  const size_t off = monolith_tmp_off(dtype, B, H, D, L, wscale ? MTP_FP8E4M3 : w_dtype, N);
+  const MonolithSpace m = monolith_space(dtype, B, H, D, L, wscale ? MTP_FP8E4M3 : w_dtype, N);
+  if (!workspace || workspace_bytes < m.least + m.tmp) return MTP_ERR_WORKSPACE;
+  // the stages take what is there before the intermediate
+  const size_t off = std::min(m.best, (workspace_bytes - m.tmp) / 256 * 256);
   void *tmp = (unsigned char *)workspace + off;
   int s = dense_attention(q, dtype, B, H, D, k, v, L, mask, mask_dtype, 0, nullptr, nullptr, scale,
                           tmp, workspace, off, stream);

@@ -214,3 +214,40 @@ def test_unaligned_query_or_output_needs_no_workspace(which, dtype):
         assert st == L.OK
         _check(out.view(B, H, D), ref, dtype)
     _check(mk.fused_causal_attention(q, k, v), ref, dtype)
+
+
+@pytest.mark.parametrize("B,H,D,L,N,dtype", [(1, 2, 128, 1000, 512, torch.float32),
+                                             (24, 12, 64, 512, 600, torch.bfloat16),
+                                             (5, 70, 64, 130, 130, torch.float16)])
+def test_monolith_needs_no_more_workspace_than_without_the_faster_plans(B, H, D, L, N, dtype):
+    """Key chunks of the decode kernel and the prompt GEMM's x * gamma are
+    taken where the workspace has room; any size from the one without them on
+    runs, a smaller one is refused."""
+    from mtp_hip import _lib as LB
+    lib = LB.load()
+    code = LB.code(dtype)
+    with LB.tuning(attn_dec=0, pg=0):
+        least = lib.mtp_tree_attn_rmsnorm_linear_workspace_bytes(code, B, H, D, L, code, N)
+    best = lib.mtp_tree_attn_rmsnorm_linear_workspace_bytes(code, B, H, D, L, code, N)
+    assert best > least
+    g = torch.Generator().manual_seed(N)
+    q = torch.randn(B, H, D, generator=g).to(dtype)
+    k, v = (torch.randn(B, H, L, D, generator=g).to(dtype) for _ in range(2))
+    W = (0.05 * torch.randn(N, D, generator=g)).to(dtype)
+    mask = (torch.rand(L, generator=g) > 0.4).float()
+    gm = 1 + 0.1 * torch.randn(D, generator=g)
+    ref = O.tree_attn_rmsnorm_linear(q, k, v, mask, W, gm)
+    dev = [t.to(DEV) for t in (q, k, v, mask, W, gm)]
+    qd, kd, vd, md, Wd, gd = (t.data_ptr() for t in dev)
+    out = torch.empty(B, H, N, dtype=dtype, device=DEV)
+    ws = torch.zeros(best + 4096, dtype=torch.uint8, device=DEV)
+    for n in (best + 4096, best, best - 1, (least + best) // 2, least, least - 1):
+        print(f"case monolith {dtype} B={B} H={H} workspace={n}", flush=True)
+        st = lib.mtp_fused_tree_attn_rmsnorm_linear(
+            qd, code, B, H, D, kd, vd, L, md, LB.F32, Wd, code, N, gd, LB.F32, None, 0, None,
+            D ** -0.5, 1e-6, out.data_ptr(), ws.data_ptr(), n, LB.stream_handle(out.device))
+        if n < least:
+            assert st == LB.ERR_WORKSPACE
+            continue
+        assert st == LB.OK
+        _check(out, ref, dtype)
