@@ -1310,7 +1310,12 @@ DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64
       int64_t nc = div ? slots / (units * div) : 1;
       nc = std::max<int64_t>(1, std::min<int64_t>({nc, blocks, (int64_t)kAttnMaxChunks}));
       int64_t cb = (blocks + nc - 1) / nc;
-      if (tune(kTuneAttnChunkBlocks) > 0) cb = std::min<int64_t>(tune(kTuneAttnChunkBlocks), blocks);
+      if (tune(kTuneAttnChunkBlocks) > 0) {
+        // a workgroup per chunk in grid.y, partials per chunk: the key keeps
+        // the bound on chunks
+        cb = std::max<int64_t>(tune(kTuneAttnChunkBlocks), (blocks + kAttnMaxChunks - 1) / kAttnMaxChunks);
+        cb = std::min(cb, blocks);
+      }
       nc = (blocks + cb - 1) / cb;
       if (nc > 1 && units > kCounterSlots) {
         nc = 1;
