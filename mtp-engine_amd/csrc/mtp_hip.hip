@@ -1275,7 +1275,7 @@ AttnPlan make_attn_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int
 // blocks of 64 keys of one (batch, head, query).
 struct DecPlan {
   bool fast = false;
-  int waves = 16, nchunks = 1, chunk_blocks = 1;
+  int waves = 0, nchunks = 1, chunk_blocks = 1;
   size_t part_off = 0, total = 0;
 };
 
@@ -1297,12 +1297,13 @@ DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64
   // past the last one of a step still fit an int
   if (B * H > (int64_t)UINT32_MAX / 1024 || Lc + Lt > INT32_MAX - (1 << 20)) return p;
   p.fast = true;
+  const int maxw = dec_max_waves(kv_fp8 ? MTP_FP8E4M3 : ct);
+  p.waves = maxw;
   const int64_t units = B * H * NQ;
   const int64_t blocks = (Lc + Lt + kAttnBlock - 1) / kAttnBlock;
-  if (blocks == 0) return p;
-  // 16 waves per CU in all: the workgroup size and chunk count with the
+  if (blocks == 0) return p;  // no key: rows of 0 / 0
+  // the waves of a CU in all: the workgroup size and chunk count with the
   // least work on the busiest CU
-  const int maxw = dec_max_waves(kv_fp8 ? MTP_FP8E4M3 : ct);
   double best = 0;
   for (int nw = maxw; nw >= 4; nw /= 2) {
     const int64_t slots = (int64_t)device_cus() * maxw / nw;

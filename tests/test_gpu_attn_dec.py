@@ -251,3 +251,22 @@ def test_monolith_needs_no_more_workspace_than_without_the_faster_plans(B, H, D,
             continue
         assert st == LB.OK
         _check(out, ref, dtype)
+
+
+@pytest.mark.parametrize("kv", ["same", "fp8"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_no_keys(D, dtype, kv, tune):
+    """An empty context runs on every K / V type, with the rows of the
+    general kernel (0 / 0)."""
+    import mtp_kernels as mk
+    q = torch.randn(2, 3, D, generator=torch.Generator().manual_seed(D)).to(dtype).to(DEV)
+    k = torch.zeros(2, 3, 0, D, dtype=torch.float8_e4m3fn if kv == "fp8" else dtype, device=DEV)
+    s = torch.ones(3, device=DEV)
+    outs = []
+    for dec in (-1, 0):
+        tune(attn_dec=dec)
+        print(f"case decode no keys {dtype} {kv} D={D} attn_dec={dec}", flush=True)
+        outs.append(mk.fused_causal_attention_fp8(q, k, k, s, s) if kv == "fp8" else
+                    mk.fused_causal_attention(q, k, k))
+    assert torch.equal(torch.isnan(outs[0]), torch.isnan(outs[1])) and bool(outs[0].isnan().all())
