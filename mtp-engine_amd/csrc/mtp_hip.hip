@@ -846,10 +846,11 @@ int launch_skp(const PlanSkp &p, SkpArgs &a, void *ws, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // Prompt GEMM plan (pg.hpp): more than 64 rows of 16-bit x, W of fp8 or the
 // same 16-bit type, whole 64-k stages. Workspace: counters (left alone),
-// x * gamma (gamma only) and the row factors.
+// x * gamma (gamma only) and the row factors of a pass, the splits' sums.
 struct PlanPg {
   bool ok = false;
   int ct = 0, wt = 0, shape = 0, S = 1, kper = 0, tiles = 0;
+  int64_t rows = 0;  // rows of a pass (prep and GEMM), all M where x * gamma fits
   bool gam = false;
   size_t xg_off = 0, rs_off = 0, part_off = 0, total = 0;
 };
@@ -868,6 +869,14 @@ struct PlanPg {
 constexpr int64_t kPgSmallBytes = (int64_t)80 << 20;
 // a launch has less than 2^32 threads in x; the prep takes 256 a row
 constexpr int64_t kPgMaxRows = (int64_t)UINT32_MAX / 256;
+// x * gamma kept at most: callers hold their workspace for good, so a longer
+// prompt goes in passes of equal rows, whole 256-row tiles, over this much of
+// it. us, one pass / passes (bf16, fp8 W): 16384 x 14336 x 8192 3180 / 3108,
+// 2920 / 2840; 32768 x 4096 x 8192 1970 / 1937, 1806 / 1779; 20000 x 1024 x
+// 4096 229 / 212, 220 / 216; where the rounds of a pass are fuller or emptier
+// than those of one launch 17000 x 512 x 4096 139 / 124, 122 / 132, and 9000
+// x 1024 x 8192 225 / 224, 189 / 215. 64 MiB: 20000 x 1024 248, 268.
+constexpr int64_t kPgXgBytes = (int64_t)128 << 20;
 
 PlanPg plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
   PlanPg p;
@@ -878,6 +887,14 @@ PlanPg plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
   if (wt != MTP_FP8E4M3 && wt != ct) return p;
   if (tune(kTunePg) == 0 || M <= 64 || N <= 0 || K <= 0 || K % kPgK != 0) return p;
   if (M > kPgMaxRows) return p;
+  p.rows = M;
+  if (gam && M * K * 2 > kPgXgBytes) {
+    const int64_t most = kPgXgBytes / (K * 2) / 256 * 256;
+    if (most == 0) return p;  // K > 262144
+    const int64_t passes = (M + most - 1) / most;
+    p.rows = ((M + passes - 1) / passes + 255) / 256 * 256;
+    M = p.rows;
+  }
   if (tune(kTuneWsVariant) >= 0 || tune(kTuneWsSplits) > 0) return p;  // sweeps of wsp
   // buffer descriptors: a tile's rows of x and of W (256 at most)
   if (256 * K * 2 >= (int64_t)1 << 31) return p;
@@ -969,43 +986,52 @@ int launch_pg(const PlanPg &p, const void *x, const float *gamma, float eps, int
   PgKernel k = pg_pick(p.ct, p.wt, p.shape, p.S > 1);
   if (!k) return MTP_ERR_DTYPE;
   unsigned char *w8 = (unsigned char *)ws;
-  a.x = x;
-  if (norm || p.gam) {
-    PgPrepKernel pk = pg_prep_pick(p.ct, p.gam);
-    if (!pk) return MTP_ERR_DTYPE;
-    PgPrepArgs pa{};
-    pa.x = x;
-    pa.gamma = gamma;
-    pa.xg = p.gam ? w8 + p.xg_off : nullptr;
-    pa.rs = (float *)(w8 + p.rs_off);
-    pa.K = a.K;
-    pa.norm = norm;
-    pa.eps = eps;
-    hipLaunchKernelGGL(pk, dim3((unsigned)a.M), dim3(256), 0, st, pa);
-    const int s = launch_status();
-    if (s != MTP_OK) return s;
-    a.rs = pa.rs;
-    if (p.gam) a.x = pa.xg;
-  }
   const PgShape sh = kPgShapes[p.shape];
   const int wb = dtype_bytes(p.wt);
   const int lds = pg_stages(sh, wb) * pg_stage_bytes(sh, wb);
-  a.gm = (a.M + sh.bm() - 1) / sh.bm();
-  a.tiles = p.tiles;
-  a.S = p.S;
-  a.kper = p.kper;
-  if (p.S > 1) {
-    a.part = (float *)(w8 + p.part_off);
-    a.ticket = (unsigned *)w8;
-  }
   const hipError_t e =
       hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) {
     note_hip_error(e);
     return MTP_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(k, dim3((unsigned)(p.tiles * p.S)), dim3((unsigned)sh.threads()), (size_t)lds, st, a);
-  return launch_status();
+  a.S = p.S;
+  a.kper = p.kper;
+  if (p.S > 1) {
+    a.part = (float *)(w8 + p.part_off);
+    a.ticket = (unsigned *)w8;
+  }
+  unsigned char *const y = (unsigned char *)a.y;
+  const int64_t M = a.M;
+  for (int64_t m0 = 0; m0 < M; m0 += p.rows) {
+    a.M = (int)std::min(p.rows, M - m0);
+    a.x = (const unsigned char *)x + m0 * a.K * 2;
+    a.y = y + m0 * a.N * 2;
+    if (norm || p.gam) {
+      PgPrepKernel pk = pg_prep_pick(p.ct, p.gam);
+      if (!pk) return MTP_ERR_DTYPE;
+      PgPrepArgs pa{};
+      pa.x = a.x;
+      pa.gamma = gamma;
+      pa.xg = p.gam ? w8 + p.xg_off : nullptr;
+      pa.rs = (float *)(w8 + p.rs_off);
+      pa.K = a.K;
+      pa.norm = norm;
+      pa.eps = eps;
+      hipLaunchKernelGGL(pk, dim3((unsigned)a.M), dim3(256), 0, st, pa);
+      const int s = launch_status();
+      if (s != MTP_OK) return s;
+      a.rs = pa.rs;
+      if (p.gam) a.x = pa.xg;
+    }
+    a.gm = (a.M + sh.bm() - 1) / sh.bm();
+    a.tiles = a.gm * ((a.N + sh.bn() - 1) / sh.bn());
+    hipLaunchKernelGGL(k, dim3((unsigned)(a.tiles * p.S)), dim3((unsigned)sh.threads()), (size_t)lds,
+                       st, a);
+    const int s = launch_status();
+    if (s != MTP_OK) return s;
+  }
+  return MTP_OK;
 }
 
 int launch_generic_linear(const void *x, int xt, const void *w, int wt, const float *wscale,

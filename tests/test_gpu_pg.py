@@ -87,3 +87,27 @@ def test_graph_replay():
         gr.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("dtype,w", TYPES)
+def test_long_prompt_in_passes(dtype, w):
+    """x * gamma above 128 MiB goes in passes of whole 256-row tiles, the last
+    one shorter and ragged: rows around the seams, against the oracle (K 512:
+    two passes, of 66048 rows and 65953)."""
+    import mtp_kernels as mk
+    M, N, K = 132001, 40, 512
+    g = torch.Generator().manual_seed(11)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    W = 0.02 * torch.randn(N, K, generator=g)
+    gm = 1 + 0.1 * torch.randn(K, generator=g)
+    print(f"case pg passes {dtype} {w} M={M}", flush=True)
+    if w == "fp8":
+        wq, ws = O.quantize_fp8_per_channel(W)
+        y = mk.fused_rmsnorm_linear_fp8(x.to(DEV), wq.to(DEV), ws.to(DEV), gamma=gm.to(DEV)).cpu()
+        ref = O.rmsnorm_linear_fp8(x, wq, ws, None, 1e-6, gamma=gm)
+    else:
+        y = mk.fused_rmsnorm_linear(x.to(DEV), W.to(dtype).to(DEV), gamma=gm.to(DEV)).cpu()
+        ref = O.rmsnorm_linear(x, W.to(dtype), None, 1e-6, 1.0, gamma=gm)
+    for rows in (slice(0, 64), slice(66000, 66100), slice(M - 64, M), slice(0, M)):
+        ok, worst = close(y[rows], ref[rows], 2e-2)
+        assert ok, f"rows {rows}: worst err/bound = {worst:.3g}"

@@ -20,3 +20,14 @@ def test_decode_attention_has_at_most_64_chunks(lib, dtype, D, keys, chunk):
         n = lib.mtp_attention_workspace_bytes(dtype, 1, 1, 3, D, 0, keys)
     most = L.MTP_COUNTER_BYTES + 3 * 64 * (D + 2) * 4
     assert n <= -(-most // 256) * 256
+
+
+@pytest.mark.parametrize("w", [L.BF16, L.FP8E4M3])
+@pytest.mark.parametrize("M,K", [(16384, 4096), (16385, 4096), (32768, 8192), (10 ** 6, 4096),
+                                 (65, 262144), (1000, 262208)])
+@pytest.mark.parametrize("N", [64, 14336])
+def test_long_prompts_keep_a_bounded_workspace(lib, M, N, K, w):
+    """x * gamma of at most 128 MiB at a time, beside the counters, the row
+    factors and the sums of K-splits (two 128 x 128 fp32 tiles per CU)."""
+    most = L.MTP_COUNTER_BYTES + (128 << 20) + 4 * M + 256 * 2 * 128 * 128 * 4 + 1024
+    assert lib.mtp_rmsnorm_linear_workspace_bytes(L.BF16, w, M, N, K) <= most
