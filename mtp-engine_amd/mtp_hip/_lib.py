@@ -195,8 +195,10 @@ def ptr(t) -> int | None:
 
 # The current stream's handle by device index, without the Stream object that
 # torch.cuda.current_stream() makes on every call (1.8 us against 0.1, twice a
-# call).
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# call). A torch built without a GPU has none: the package still imports there
+# (and current_stream() raises what torch says).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                      lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _index(device: torch.device) -> int:

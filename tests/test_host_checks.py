@@ -1,9 +1,14 @@
 """Host-side guards of the Python shim (CPU): tensors that are not on a HIP
 device, or whose shapes disagree, are refused before any library call, and
 CachedLinear's cached views follow its parameters through .to()."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
+from conftest import PKG
 from mtp_hip import ops
 
 
@@ -42,3 +47,21 @@ def test_cached_linear_follows_module_moves():
     lin = lin.to(torch.float64)
     assert lin._w.dtype == torch.float64 and lin._w.data_ptr() == lin.weight.data_ptr()
     assert lin._b.data_ptr() == lin.bias.data_ptr()
+
+
+def test_package_imports_on_a_torch_without_a_gpu():
+    """A CPU-only torch has no raw-stream function: every module imports and a
+    host tensor is refused as ever."""
+    code = ("import torch\n"
+            "if hasattr(torch._C, '_cuda_getCurrentRawStream'):\n"
+            "    del torch._C._cuda_getCurrentRawStream\n"
+            "import mtp_hip, mtp_kernels, mtp_fused_verify\n"
+            "from mtp_hip import ops\n"
+            "try:\n"
+            "    ops.rmsnorm_linear(torch.randn(4, 64), torch.randn(32, 64))\n"
+            "except RuntimeError as e:\n"
+            "    assert 'HIP device' in str(e)\n"
+            "    print('refused')\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
+                       env={**os.environ, "PYTHONPATH": PKG})
+    assert r.returncode == 0 and "refused" in r.stdout, r.stderr
