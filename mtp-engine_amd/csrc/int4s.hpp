@@ -380,15 +380,16 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
   };
 
   // ---- the waves' sums in wave order (first unit's and second unit's
-  // columns), row factor, output: thread (tile, column, rows 4 q .. 4 q + 3).
-  // The sums hold x * gamma before the row factor, so they can leave fp32's
-  // range where the output does not (a row whose squares overflow has the
-  // factor 0 and is 0; a huge gamma): an output that is not finite, of a row
-  // without NaN, is computed again in the order of the definition.
+  // columns), row factor, output: thread (tile, column, rows 4 q .. 4 q + 3)
   constexpr int RQ = 2 * MH;
   const int nout = ntl * 8 * RQ;
-  for (int i0 = 64 * wave; i0 < nout; i0 += 64 * nw) {
-    const int i = min(i0 + lane, nout - 1);
+  auto row_factor = [&](int m) {
+    float s2 = 0.f;
+    for (int q = 0; q < nw; ++q) s2 += MH == 1 ? s_ss[q][m] + s_ss[q][m + 8] : s_ss[q][m];
+    return 1.0f / sqrtf(s2 / (float)K + a.eps);
+  };
+  bool bad = false;  // an output that is not finite
+  for (int i = th; i < nout; i += 64 * nw) {
     const int t = i / (8 * RQ), rem = i - t * 8 * RQ, q4 = rem >> 3, col = rem & 7;
     const int n = n0 + t * 8 + col;
     const int s0 = col + 16 * q4, s1 = 8 + col + 16 * q4;
@@ -400,22 +401,38 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = 4 * q4 + r;
-      const bool on = i0 + lane < nout && m < a.M && n < a.N;
-      float f = 1.f;
-      if (a.norm) {
-        float s2 = 0.f;
-        for (int q = 0; q < nw; ++q) s2 += MH == 1 ? s_ss[q][m] + s_ss[q][m + 8] : s_ss[q][m];
-        f = 1.0f / sqrtf(s2 / (float)K + a.eps);
+      if (m >= a.M || n >= a.N) continue;
+      const float y = v[r] * (a.norm ? row_factor(m) : 1.f);
+      bad |= !(fabsf(y) < INFINITY);
+      ((uint16_t *)a.y)[(int64_t)m * a.N + n] = (uint16_t)pack2<XT>(y, 0.f);
+    }
+  }
+  // The sums hold x * gamma before the row factor, so they can leave fp32's
+  // range where the output does not (a row whose squares overflow has the
+  // factor 0 and is 0; a huge gamma). Outputs that are not finite, of rows
+  // without NaN, are computed again in the order of the definition, by the
+  // wave that wrote them.
+  if (!a.norm || __builtin_expect(__ballot(bad) == 0, 1)) return;
+#pragma unroll 1
+  for (int i0 = 64 * wave; i0 < nout; i0 += 64 * nw) {
+    const int i = min(i0 + lane, nout - 1);
+    const int t = i / (8 * RQ), rem = i - t * 8 * RQ, n = n0 + t * 8 + (rem & 7);
+#pragma unroll 1
+    for (int r = 0; r < 4; ++r) {
+      const int m = 4 * (rem >> 3) + r;
+      float f = 0.f;
+      bool again = i0 + lane < nout && m < a.M && n < a.N;
+      if (again) {
+        f = row_factor(m);
+        again = f == f &&
+                !(fabsf(load_as_f32(a.y, XT, (int64_t)m * a.N + n)) < INFINITY);
       }
-      float y = v[r] * f;
-      if (a.norm) {
-        for (uint64_t bad = __ballot(on && f == f && !(fabsf(y) < INFINITY)); bad; bad &= bad - 1) {
-          const int l = __builtin_ctzll(bad);
-          const float z = direct(__shfl(m, l, 64), __shfl(n, l, 64), __shfl(f, l, 64));
-          y = lane == l ? z : y;
-        }
+#pragma unroll 1
+      for (uint64_t todo = __ballot(again); todo; todo &= todo - 1) {
+        const int l = __builtin_ctzll(todo);
+        const float z = direct(__shfl(m, l, 64), __shfl(n, l, 64), __shfl(f, l, 64));
+        if (lane == l) ((uint16_t *)a.y)[(int64_t)m * a.N + n] = (uint16_t)pack2<XT>(z, 0.f);
       }
-      if (on) ((uint16_t *)a.y)[(int64_t)m * a.N + n] = (uint16_t)pack2<XT>(y, 0.f);
     }
   }
 }
