@@ -8,7 +8,8 @@
 // traffic between tiles: per tile one 16-byte weight load per lane (8 rows x
 // 128 contiguous bytes an instruction; 16 rows x 64 bytes, the plain MFMA
 // layout, took 41.5 us where this takes 36.5) and the scales, a ring of R
-// tiles ahead (128 KB of W in flight per CU).
+// tiles with R - 1 ahead (32 to 96 KB of W in flight per CU; 80 at groups of
+// 128 with their scales in LDS, 56 above 8 rows).
 //   * x: the wave loads its chunk's rows as they are, takes x * gamma, scales
 //     every row of a unit by the power of two that brings its largest entry
 //     into [2^14, 2^15] and rounds to fp16 (11 bits; undone exactly on the
@@ -31,7 +32,7 @@
 // Measured, 8 rows, N 28672, K 8192, groups of 128, norm and gamma: 48.4 ->
 // 30.0 us a call (4.1 TB/s) against the prep launch and LDS-staged kernel of
 // more rows; N 14336, K 4096: 24.8 -> 13.3. Vector work (decode, x) is half of
-// the time. The ring is a tile shorter with LDS scales (128 registers).
+// the time.
 #pragma once
 
 #include "int4s_args.hpp"
@@ -73,8 +74,17 @@ __global__ void __launch_bounds__(64 * i4s_max_waves(MH)) int4s_kernel(const I4s
   constexpr bool SVEC = SM == kI4sScaleVec, SLDS = SM == kI4sScaleLds;
   // registers of a unit's scales: whole pieces of the row, or one each
   constexpr int SR = SLDS ? 1 : !SVEC ? NG : NG * SB < 4 ? 1 : NG * SB / 4;
-  // ring: tiles in flight (128 registers up to 8 rows)
-  constexpr int R = MH == 2 ? 8 : SLDS ? (NG == 4 ? 5 : 6) : SR == 1 ? 7 : SR == 2 ? 5 : 4;
+  // ring: R - 1 tiles of 1 KB a wave in flight, as deep as no form spills (128
+  // registers up to 8 rows; scales take their share of a slot, groups below
+  // 128 more sums). Deeper rings with 1 to 5 registers spilled, us: groups of
+  // 32 8 x 14336 x 4096 15.9 / 13.6 here, 1 x 8192 x 8192 17.6 / 14.6, 8 x
+  // 28672 x 8192 43.5 / 41.5; of 64 14.3 / 13.6, 14.8 / 14.4, 36.0 / 36.2.
+  constexpr int R = MH == 2                ? 8
+                    : SLDS                 ? (NG == 1 ? 6 : NG == 2 ? 5 : 4)
+                    : SR == 1              ? 7
+                    : SR == 2 && NG == 4   ? 4
+                    : SR == 2              ? 5
+                                           : 3;
   constexpr int SPG = GRP / 32;  // MFMA k-steps per group
   constexpr int AL = 32 * MH;    // lanes of a tile's sums kept (8 or 16 rows)
   extern __shared__ __attribute__((aligned(16))) f32x4 s_acc[];  // [wave][tile][AL], gamma [K]

@@ -1608,9 +1608,9 @@ bool launch_int4s(const void *x, int xdt, int64_t M, int64_t K, const uint8_t *p
   a.nt = (int)std::min<int64_t>({kI4sMaxTiles, fit, (tiles + device_cus() - 1) / device_cus()});
   const int64_t grid = (tiles + a.nt - 1) / a.nt;
   // Scale rows through LDS where they are whole 16-byte pieces and fit beside
-  // the sums (us, 2-byte loads / LDS: M 8 N 28672 K 8192 G 128 31.5 / 30.0,
-  // M 5 N 4096 K 4096 G 32 11.5 / 11.0, M 12 N 20000 K 2048 G 64 fp32 13.9 /
-  // 12.6, M 2 N 14336 K 4096 G 128 13.7 / 13.3)
+  // the sums (us, own loads / LDS: M 8 N 28672 K 8192 G 128 34.6 / 31.8, G 32
+  // 37.4 / 37.0, M 5 N 4096 K 4096 G 32 9.9 / 9.3, M 12 N 20000 K 2048 G 64
+  // fp32 13.5 / 12.6, M 2 N 14336 K 4096 G 128 13.0 / 12.7)
   const int64_t srow = ng * sb, sl = a.nt * 8 * (srow + 4);
   const bool slds = tune(kTuneInt4s) != 2 && srow % 16 == 0 && aligned16(scales) &&
                     tb * a.nt + gb + sl <= kLds &&
