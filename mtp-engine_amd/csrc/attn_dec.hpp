@@ -278,10 +278,11 @@ __global__ void __launch_bounds__(64 * dec_max_waves(KT)) attn_dec_kernel(const 
   const int64_t oo = (int64_t)b * a.o_sb + (int64_t)qi * a.o_sn + (int64_t)h * a.o_sh;
   // (M, L, O[d]) over the first n entries of s_ml / s_o, every LDS read in
   // flight at once
-  auto merge_entries = [&](int n, int d, float &M, float &L, float &O) {
-    float em[MAXW], el[MAXW], eo[MAXW];
+  auto merge_first = [&](auto most, int n, int d, float &M, float &L, float &O) {
+    constexpr int MOST = decltype(most)::value;
+    float em[MOST], el[MOST], eo[MOST];
 #pragma unroll
-    for (int w = 0; w < MAXW; ++w) {
+    for (int w = 0; w < MOST; ++w) {
       const int ww = min(w, n - 1);
       em[w] = s_ml[ww][0];
       el[w] = s_ml[ww][1];
@@ -289,18 +290,22 @@ __global__ void __launch_bounds__(64 * dec_max_waves(KT)) attn_dec_kernel(const 
     }
     M = em[0];
 #pragma unroll
-    for (int w = 1; w < MAXW; ++w) M = fmaxf(M, em[w]);
+    for (int w = 1; w < MOST; ++w) M = fmaxf(M, em[w]);
     const float ref = M == -INFINITY ? 0.f : M;
     L = 0.f;
     O = 0.f;
 #pragma unroll
-    for (int w = 0; w < MAXW; ++w) {
+    for (int w = 0; w < MOST; ++w) {
       const float e = __builtin_amdgcn_exp2f(em[w] - ref);
       if (w < n) {
         L = fmaf(el[w], e, L);
         O = fmaf(eo[w], e, O);
       }
     }
+  };
+  auto merge_entries = [&](int n, int d, float &M, float &L, float &O) {
+    if (n <= 4) merge_first(std::integral_constant<int, 4>{}, n, d, M, L, O);
+    else merge_first(std::integral_constant<int, MAXW>{}, n, d, M, L, O);
   };
   if (th < D) {
     float M, L, O;

@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 
@@ -1305,6 +1306,66 @@ struct DecPlan {
   size_t part_off = 0, total = 0;
 };
 
+// Chunks of attn_chunk_blocks blocks where the key is set: a workgroup per
+// chunk in grid.y and partials per chunk, so it keeps the bound on chunks.
+int64_t dec_chunk_blocks(int64_t cb, int64_t blocks) {
+  if (tune(kTuneAttnChunkBlocks) > 0)
+    cb = std::max<int64_t>(tune(kTuneAttnChunkBlocks), (blocks + kAttnMaxChunks - 1) / kAttnMaxChunks);
+  return std::min(cb, blocks);
+}
+
+// Waves and chunks of a 16-bit single query at head dim 64 or 128, which the
+// MFMA kernel takes too and is hard to beat at a few hundred keys: the least
+// of a model of the launch, in us. A term per wave of a workgroup; a round of
+// workgroups (16 waves to a CU) is its ends and the root of the squares of its
+// three bounds, the chain of a wave's steps and the CU's and the chip's rate
+// for the keys that it reads; chunks cost their merge. Fitted to bf16, dense
+// and paged, D 64 and 128, 1 .. 384 heads, 32 .. 4096 keys, K / V from HBM (676
+// sizes x 3 to 30 plans): 1 % off the best plan in the mean, 12 % at most (the
+// rule of the other calls 17 %, 2 x at most), and above 64 keys at most 3 %
+// slower than the MFMA kernel (8 % with K / V in the caches; 64 keys and fewer
+// at D 64 take it 4.1 us and this kernel 4.8). K / V in the caches, us, MFMA
+// kernel / the other rule / here: 16 heads, D 64, 512 keys 6.8 / 8.6 / 7.2, 1024
+// keys 8.1 / 8.8 / 7.8, D 128, 512 keys 7.7 / 9.4 / 7.8; 384 heads, D 64, 128
+// keys 6.4 / 9.6 / 5.7.
+void plan_dec_16bit(DecPlan &p, int64_t units, int64_t keys, int64_t D) {
+  constexpr double kWave = 0.0267, kEnds = 1.44, kStep = 0.46;
+  constexpr double kCuRate = 57.7e3, kChipRate = 6.85e6;  // bytes per us
+  constexpr double kMerge = 0.96, kMergeChunk = 0.066;
+  const int maxw = dec_max_waves(MTP_BF16);
+  const int64_t blocks = (keys + kAttnBlock - 1) / kAttnBlock;
+  const int64_t step = 64 / (D / 8) * kDecLoads;  // keys of a wave's step
+  double best = 0;
+  for (int nw = maxw; nw >= 4; nw /= 2) {
+    const int64_t slots = (int64_t)device_cus() * maxw / nw;
+    for (int64_t want : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+      int64_t cb = dec_chunk_blocks((blocks + want - 1) / want, blocks);
+      int64_t nc = (blocks + cb - 1) / cb;
+      if (nc > 1 && units > kCounterSlots) {
+        nc = 1;
+        cb = blocks;
+      }
+      const int64_t ck = std::min(keys, cb * kAttnBlock), groups = units * nc;
+      const double bytes = (double)(ck * D * 4);  // K and V of a workgroup
+      const int64_t percu = std::min<int64_t>(maxw / nw, (groups + device_cus() - 1) / device_cus());
+      const double chain = kStep * (double)((ck + step * nw - 1) / (step * nw));
+      const double cu = (double)percu * bytes / kCuRate;
+      const double chip = (double)std::min(groups, slots) * bytes / kChipRate;
+      const double cost = kWave * nw +
+                          (double)((groups + slots - 1) / slots) *
+                              (kEnds + std::sqrt(chain * chain + cu * cu + chip * chip)) +
+                          (nc > 1 ? kMerge + kMergeChunk * (double)nc : 0);
+      if (best == 0 || cost < best) {
+        best = cost;
+        p.waves = nw;
+        p.nchunks = (int)nc;
+        p.chunk_blocks = (int)cb;
+      }
+      if (want >= blocks || units > kCounterSlots) break;
+    }
+  }
+}
+
 // What a merge of chunks costs (partials through the device coherence point,
 // arrival ticket, the last workgroup's loads), in blocks of 64 keys at the
 // rate a CU reads them when the whole chip reads (about 1.2 us for bf16 at
@@ -1313,23 +1374,9 @@ struct DecPlan {
 // in one chunk, 100.1 in 4.
 constexpr double kDecMergeBlocks = 2.5, kDecMergeChunk = 0.2;
 
-DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64_t Lc, int64_t Lt,
-                      bool kv_fp8) {
-  DecPlan p;
-  if (D != 64 && D != 128 && D != 256) return p;
-  const bool mfma = (ct == MTP_BF16 || ct == MTP_F16) && D != 256 && NQ > 1 && NQ <= 64 && !kv_fp8;
-  if (mfma || tune(kTuneAttnDec) == 0) return p;
-  // launches of 1024 threads a workgroup end below 2^32 threads in x; keys
-  // past the last one of a step still fit an int
-  if (B * H > (int64_t)UINT32_MAX / 1024 || Lc + Lt > INT32_MAX - (1 << 20)) return p;
-  p.fast = true;
-  const int maxw = dec_max_waves(kv_fp8 ? MTP_FP8E4M3 : ct);
-  p.waves = maxw;
-  const int64_t units = B * H * NQ;
-  const int64_t blocks = (Lc + Lt + kAttnBlock - 1) / kAttnBlock;
-  if (blocks == 0) return p;  // no key: rows of 0 / 0
-  // the waves of a CU in all: the workgroup size and chunk count with the
-  // least work on the busiest CU
+// The other calls: the waves of a CU in all, the workgroup size and chunk
+// count with the least work on the busiest CU.
+void plan_dec_other(DecPlan &p, int64_t units, int64_t blocks, int maxw) {
   double best = 0;
   for (int nw = maxw; nw >= 4; nw /= 2) {
     const int64_t slots = (int64_t)device_cus() * maxw / nw;
@@ -1337,12 +1384,7 @@ DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64
       int64_t nc = div ? slots / (units * div) : 1;
       nc = std::max<int64_t>(1, std::min<int64_t>({nc, blocks, (int64_t)kAttnMaxChunks}));
       int64_t cb = (blocks + nc - 1) / nc;
-      if (tune(kTuneAttnChunkBlocks) > 0) {
-        // a workgroup per chunk in grid.y, partials per chunk: the key keeps
-        // the bound on chunks
-        cb = std::max<int64_t>(tune(kTuneAttnChunkBlocks), (blocks + kAttnMaxChunks - 1) / kAttnMaxChunks);
-        cb = std::min(cb, blocks);
-      }
+      cb = dec_chunk_blocks(cb, blocks);
       nc = (blocks + cb - 1) / cb;
       if (nc > 1 && units > kCounterSlots) {
         nc = 1;
@@ -1361,6 +1403,27 @@ DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64
       }
     }
   }
+}
+
+DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64_t Lc, int64_t Lt,
+                      bool kv_fp8) {
+  DecPlan p;
+  if (D != 64 && D != 128 && D != 256) return p;
+  const bool mfma = (ct == MTP_BF16 || ct == MTP_F16) && D != 256 && NQ > 1 && NQ <= 64 && !kv_fp8;
+  if (mfma || tune(kTuneAttnDec) == 0) return p;
+  // launches of 1024 threads a workgroup end below 2^32 threads in x; keys
+  // past the last one of a step still fit an int
+  if (B * H > (int64_t)UINT32_MAX / 1024 || Lc + Lt > INT32_MAX - (1 << 20)) return p;
+  p.fast = true;
+  const int maxw = dec_max_waves(kv_fp8 ? MTP_FP8E4M3 : ct);
+  p.waves = maxw;
+  const int64_t units = B * H * NQ;
+  const int64_t blocks = (Lc + Lt + kAttnBlock - 1) / kAttnBlock;
+  if (blocks == 0) return p;  // no key: rows of 0 / 0
+  if ((ct == MTP_BF16 || ct == MTP_F16) && D != 256 && NQ == 1 && !kv_fp8)
+    plan_dec_16bit(p, units, Lc + Lt, D);
+  else
+    plan_dec_other(p, units, blocks, maxw);
   if (p.nchunks > 1) {
     p.part_off = kCounterBytes;
     p.total = kCounterBytes + align_up((size_t)units * p.nchunks * (D + 2) * 4, 256);

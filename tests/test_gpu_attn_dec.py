@@ -270,3 +270,18 @@ def test_no_keys(D, dtype, kv, tune):
         outs.append(mk.fused_causal_attention_fp8(q, k, k, s, s) if kv == "fp8" else
                     mk.fused_causal_attention(q, k, k))
     assert torch.equal(torch.isnan(outs[0]), torch.isnan(outs[1])) and bool(outs[0].isnan().all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,L,D", [(2, 8, 448, 64), (12, 1, 192, 128), (48, 8, 96, 64),
+                                     (1, 3, 3000, 128), (9, 11, 700, 128), (520, 8, 130, 64)])
+def test_planned_waves_and_chunks(B, H, L, D, dtype):
+    """Few and many heads at some hundred keys: workgroups of 4, 8 and 16
+    waves, in one chunk and several."""
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(L)
+    q = torch.randn(B, H, D, generator=g).to(dtype)
+    k, v = (torch.randn(B, H, L, D, generator=g).to(dtype) for _ in range(2))
+    print(f"case decode planned {dtype} B={B} H={H} L={L} D={D}", flush=True)
+    out = mk.fused_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV))
+    _check(out, O.causal_attention(q, k, v), dtype)
