@@ -1086,10 +1086,11 @@ int rmsnorm_linear_impl(const void *x, int xt, int64_t M, int64_t K, const void 
   // a wave round more than the tiled kernel's: 2.2e-7 against 1.8e-7 at K
   // 4096) and at most two workgroups per CU in all (48 rows, us, tiled / this:
   // K 1024 N 970 19.6 / 7.5, N 4096 18.8 / 13.8, N 8192 20.9 / 26.7; K 256 N
-  // 4096 14.4 / 8.8, N 8192 14.7 / 15.8)
+  // 4096 14.4 / 8.8, N 8192 14.7 / 15.8), a second one from K 128 on (N 2500: K
+  // 64 7.7 / 8.4, K 128 10.2 / 8.8)
   const int64_t sf_blocks = (N + 15) / 16;
-  const bool sf_rows =
-      M <= 32 || (M <= kSf32MaxRows && K <= 1536 && sf_blocks <= device_cus());
+  const bool sf_rows = M <= 32 || (M <= kSf32MaxRows && K <= 1536 && sf_blocks <= device_cus() &&
+                                   (2 * sf_blocks <= device_cus() || K >= 128));
   if (xt == MTP_F32 && wt == MTP_F32 && !wscale && tune(kTuneSf32) != 0 && sf_rows &&
       K >= 16 && K <= kSf32StreamMaxK && K % 16 == 0 && aligned && (!gamma || gt == MTP_F32) &&
       tune(kTuneWsVariant) < 0 && tune(kTuneWsSplits) <= 0) {

@@ -28,3 +28,24 @@ def test_rows_33_to_64(M, N, K, gamma, bias):
                                 gamma=gm.to(DEV) if gamma else None)
     ok, worst = close(y, O.rmsnorm_linear(x, W, b, 1e-6, 1.0, gamma=gm), 1e-5)
     assert ok, f"worst err/bound = {worst:.3g}"
+
+
+@pytest.mark.parametrize("M", [33, 48])
+@pytest.mark.parametrize("N,K,tiled", [(2500, 64, True), (2064, 112, True), (2048, 64, False),
+                                       (2500, 128, False)])
+def test_short_rows_of_many_columns_keep_the_tiled_kernel(M, N, K, tiled, tune):
+    """A second workgroup per CU pays from K 128 on: below, the planned call
+    has the bits of the tiled kernel."""
+    import mtp_kernels as mk
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g)
+    W = 0.02 * torch.randn(N, K, generator=g)
+    gm = 1 + 0.1 * torch.randn(K, generator=g)
+    args = [t.to(DEV) for t in (x, W)]
+    print(f"case sf32 short rows M={M} N={N} K={K}", flush=True)
+    y = mk.fused_rmsnorm_linear(*args, gamma=gm.to(DEV))
+    ok, worst = close(y, O.rmsnorm_linear(x, W, None, 1e-6, 1.0, gamma=gm), 1e-5)
+    assert ok, f"worst err/bound = {worst:.3g}"
+    tune(sf32=0)
+    if tiled:
+        assert torch.equal(y, mk.fused_rmsnorm_linear(*args, gamma=gm.to(DEV)))
