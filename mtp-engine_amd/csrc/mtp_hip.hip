@@ -879,6 +879,22 @@ constexpr int64_t kPgMaxRows = (int64_t)UINT32_MAX / 256;
 // x 1024 x 8192 225 / 224, 189 / 215. 64 MiB: 20000 x 1024 248, 268.
 constexpr int64_t kPgXgBytes = (int64_t)128 << 20;
 
+// A thousand rows and more of few columns stay on the row-chunk kernel: there
+// is little to multiply, so the prep's pass over x (with gamma) and x through
+// LDS cost more than they save. us, row-chunk / prompt GEMM: fp8, gamma, N 64,
+// K 4096 2400 rows 18.8 / 20.8, 4096 rows 19.5 / 27.4, N 256 4096 rows 30.0 /
+// 34.5 (N 320 to 512 either way by up to 20 %); bf16, gamma, N 64, K 8192 3200
+// rows 29.0 / 35.0 (N 128 37.3 / 44.2, but 1200 rows 28.1 / 22.9); without gamma
+// fp8, N 64, K 8192 3200 rows 23.5 / 27.4, bf16, N 16, K 4096 16.2 / 20.2 (N 64
+// 19.3 / 20.5, K 8192 28.9 / 27.2).
+bool pg_too_narrow(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
+  const bool fp8 = wt == MTP_FP8E4M3;
+  if (tune(kTunePg) > 0) return false;
+  const bool narrow = gam ? M >= 1000 && M * K >= 3200000 && N <= (fp8 ? 256 : 112)
+                          : M >= 2000 && M * K >= 10000000 && N <= (fp8 ? 128 : 16);
+  return narrow && make_plan_x(ct, wt, M, N, K, gam).ok;
+}
+
 PlanPg plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
   PlanPg p;
   p.ct = ct;
@@ -887,7 +903,7 @@ PlanPg plan_pg(int ct, int wt, int64_t M, int64_t N, int64_t K, bool gam) {
   if (ct != MTP_BF16 && ct != MTP_F16) return p;
   if (wt != MTP_FP8E4M3 && wt != ct) return p;
   if (tune(kTunePg) == 0 || M <= 64 || N <= 0 || K <= 0 || K % kPgK != 0) return p;
-  if (M > kPgMaxRows) return p;
+  if (M > kPgMaxRows || pg_too_narrow(ct, wt, M, N, K, gam)) return p;
   p.rows = M;
   if (gam && M * K * 2 > kPgXgBytes) {
     const int64_t most = kPgXgBytes / (K * 2) / 256 * 256;

@@ -111,3 +111,13 @@ def test_long_prompt_in_passes(dtype, w):
     for rows in (slice(0, 64), slice(66000, 66100), slice(M - 64, M), slice(0, M)):
         ok, worst = close(y[rows], ref[rows], 2e-2)
         assert ok, f"rows {rows}: worst err/bound = {worst:.3g}"
+
+
+@pytest.mark.parametrize("dtype,w", TYPES)
+@pytest.mark.parametrize("M,N,K,gamma", [(1000, 100, 3200, True), (999, 100, 3264, True),
+                                         (1100, 113, 3200, True), (2500, 16, 4096, False),
+                                         (1300, 257, 2496, True)])
+def test_many_rows_of_few_columns(M, N, K, gamma, dtype, w):
+    """Both sides of the line to the row-chunk kernel."""
+    print(f"case pg narrow {dtype} {w} M={M} N={N} K={K} {gamma}", flush=True)
+    _case(M, N, K, dtype, w, gamma=gamma)

@@ -31,3 +31,15 @@ def test_long_prompts_keep_a_bounded_workspace(lib, M, N, K, w):
     factors and the sums of K-splits (two 128 x 128 fp32 tiles per CU)."""
     most = L.MTP_COUNTER_BYTES + (128 << 20) + 4 * M + 256 * 2 * 128 * 128 * 4 + 1024
     assert lib.mtp_rmsnorm_linear_workspace_bytes(L.BF16, w, M, N, K) <= most
+
+
+@pytest.mark.parametrize("w", [L.BF16, L.FP8E4M3])
+@pytest.mark.parametrize("M,N,K,narrow", [(4096, 64, 4096, True), (1000, 100, 3200, True),
+                                          (999, 64, 4096, False), (4096, 64, 768, False),
+                                          (4096, 512, 4096, False)])
+def test_many_rows_of_few_columns_stay_on_the_row_chunk_kernel(lib, w, M, N, K, narrow):
+    """Their workspace has no room for x * gamma of every row."""
+    both = lib.mtp_rmsnorm_linear_workspace_bytes(L.BF16, w, M, N, K)
+    assert (both < M * K * 2) == narrow
+    with L.tuning(pg=0):
+        assert both >= lib.mtp_rmsnorm_linear_workspace_bytes(L.BF16, w, M, N, K)
