@@ -69,24 +69,85 @@ def test_planned(M, N, K, dtype, w, gamma, bias, norm):
     _case(M, N, K, dtype, w, gamma, bias, norm)
 
 
-def test_graph_replay():
-    """Prep, splits and arrival counts replay; eager calls in between."""
+def _planned_splits(M, N, K, wcode):
+    """Whether the plan of a bf16 call splits K: its partials are then part of
+    the workspace asked for."""
+    from mtp_hip import _lib as L
+    lib = L.load()
+    planned = lib.mtp_rmsnorm_linear_workspace_bytes(L.BF16, wcode, M, N, K)
+    with L.tuning(pg_splits=1):
+        return planned > lib.mtp_rmsnorm_linear_workspace_bytes(L.BF16, wcode, M, N, K)
+
+
+@pytest.mark.parametrize("w", ["same", "fp8"])
+def test_planned_splits(w):
+    """A size whose plan splits K, with the same bits on a repeat."""
+    from mtp_hip import _lib as L
+    assert _planned_splits(128, 1000, 4096, L.FP8E4M3 if w == "fp8" else L.BF16)
+    print(f"case pg planned splits {w}", flush=True)
+    a = _case(128, 1000, 4096, torch.bfloat16, w)
+    assert torch.equal(a, _case(128, 1000, 4096, torch.bfloat16, w))
+
+
+@pytest.mark.parametrize("M,N,K,splits", [(70, 300, 2048, False), (128, 1000, 4096, True)])
+def test_graph_replay(M, N, K, splits):
+    """Prep and GEMM replay, without K-splits and with their partials and
+    arrival counts; eager calls in between."""
     import mtp_kernels as mk
+    from mtp_hip import _lib as L
+    assert _planned_splits(M, N, K, L.BF16) == splits
     g = torch.Generator().manual_seed(9)
-    W = (0.02 * torch.randn(300, 2048, generator=g)).to(torch.bfloat16).to(DEV)
-    x = torch.randn(70, 2048, generator=g).to(torch.bfloat16).to(DEV)
-    gm = (1 + 0.1 * torch.randn(2048, generator=g)).to(DEV)
+    W = (0.02 * torch.randn(N, K, generator=g)).to(torch.bfloat16).to(DEV)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    gm = (1 + 0.1 * torch.randn(K, generator=g)).to(DEV)
     mk.fused_rmsnorm_linear(x, W, gamma=gm)
     torch.cuda.synchronize()
     gr = torch.cuda.CUDAGraph()
     with torch.cuda.graph(gr):
         y = mk.fused_rmsnorm_linear(x, W, gamma=gm)
     for i in range(4):
-        x.copy_(torch.randn(70, 2048, generator=g).to(torch.bfloat16))
+        x.copy_(torch.randn(M, K, generator=g).to(torch.bfloat16))
         ref = mk.fused_rmsnorm_linear(x, W, gamma=gm)
         gr.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("dtype,w", TYPES)
+@pytest.mark.parametrize("splits", [1, 4])
+def test_non_finite_x_and_gamma(splits, dtype, w, tune):
+    """inf and NaN in x stay in their rows, an infinite gamma reaches every
+    row, as in the oracle."""
+    import mtp_kernels as mk
+    tune(pg=13, pg_splits=splits)
+    g = torch.Generator().manual_seed(12)
+    M, N, K = 90, 70, 1024
+    x = torch.randn(M, K, generator=g).to(dtype)
+    x[3, 5], x[64, 1000], x[89, 0] = float("inf"), float("nan"), float("-inf")
+    W = 0.02 * torch.randn(N, K, generator=g)
+    gm = 1 + 0.1 * torch.randn(K, generator=g)
+    inf_gamma = gm.clone()
+    inf_gamma[77] = float("inf")
+    if w == "fp8":
+        wq, ws = O.quantize_fp8_per_channel(W)
+        dev = [t.to(DEV) for t in (x, wq, ws)]
+    else:
+        dev = [x.to(DEV), W.to(dtype).to(DEV)]
+    for gamma in (gm, inf_gamma):
+        print(f"case pg non-finite {dtype} {w} S={splits}", flush=True)
+        if w == "fp8":
+            y = mk.fused_rmsnorm_linear_fp8(*dev, gamma=gamma.to(DEV)).cpu()
+            ref = O.rmsnorm_linear_fp8(x, wq, ws, None, 1e-6, gamma=gamma)
+        else:
+            y = mk.fused_rmsnorm_linear(*dev, gamma=gamma.to(DEV)).cpu()
+            ref = O.rmsnorm_linear(x, W.to(dtype), None, 1e-6, 1.0, gamma=gamma)
+        assert torch.equal(torch.isnan(y), torch.isnan(ref))
+        assert torch.equal(torch.isinf(y), torch.isinf(ref))
+        f = torch.isfinite(ref)
+        assert bool((y[~f & ~torch.isnan(ref)] == ref[~f & ~torch.isnan(ref)]).all())
+        if bool(f.any()):
+            ok, worst = close(y[f], ref[f], 2e-2)
+            assert ok, f"worst err/bound = {worst:.3g}"
 
 
 @pytest.mark.parametrize("dtype,w", TYPES)
