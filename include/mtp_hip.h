@@ -278,8 +278,10 @@ int mtp_noalloc_init(void);
  * eager); for tests and tuning. Returns one of:
  *   MTP_VERIFY_ROUTE_STREAM        persistent W-streaming kernel (one dtype
  *                                  for hidden and W: BF16 / F16 / F32; any
- *                                  bias; K * element bytes % 512 == 0;
- *                                  16-byte aligned rows)
+ *                                  bias; 16-byte aligned rows; K * element
+ *                                  bytes % 512 == 0, or % 128 == 0 and at
+ *                                  least 1024: these calls still ask for the
+ *                                  column-group kernel's workspace)
  *   MTP_VERIFY_ROUTE_COLUMN_GROUP  column-group streaming kernel
  *   MTP_VERIFY_ROUTE_GENERIC       any dtypes, K and alignment
  * or a negative status.

@@ -59,7 +59,9 @@ int attn2_lds_bytes();
 void (*attn_generic())(AttnArgs, int, int);
 // Decode kernel (attn_dec.hpp) for K / V of type kt at head dim 64, 128 or
 // 256, with (ctx) or without a paged context; null for other shapes. Grid
-// (B * H, nchunks, NQ), 64 .. 1024 threads.
+// (B * H, nchunks, NQ); whole waves, no fewer threads than D (thread d < D
+// writes output d) and at most 64 * dec_max_waves(kt): the plans take 256 ..
+// 1024, fp8 256 .. 512.
 void (*attn_dec_pick(int kt, int d, bool ctx))(AttnArgs, int);
 // Fallback for 256 < D <= kAttnWideMaxD (one workgroup per query), or null.
 constexpr int kAttnWideMaxD = 8192;

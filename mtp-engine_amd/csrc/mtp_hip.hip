@@ -863,9 +863,11 @@ struct PlanPg {
 //  * the copies of all workgroups at the rate the L2s sustain (15 TB/s; 22
 //    while x and W together stay below 80 MB),
 // plus the hand-over of splits. Fitted to 32 sizes x 14 shapes, M 90 .. 2048,
-// N 600 .. 14336, K 512 .. 4096: its picks are 0 .. 12 % off the best shape.
+// N 600 .. 14336, K 512 .. 4096: its picks are 0 .. 12 % off the best shape
+// there; over 592 calls of M 65 .. 3200, N 64 .. 14336, K 512 .. 8192 4 % in the
+// mean, 64 of them more than 12 % (100 x 14336 x 4096 bf16 67 us, 4-wave {2, 4} 40).
 // bf16, us: 2048 x 14336 x 4096 on {7, 4} 200 (whole rounds of 256 tiles;
-// {8, 4} 203, {4, 4} 4-wave 272), 517 x 14336 on {6, 3} 67 ({8, 4} 92),
+// {8, 4} 203, {4, 4} 4-wave 272), fp8 517 x 14336 on {6, 3} 61 ({8, 4} 92),
 // 128 x 1000 x 4096 on 4 splits of {2, 1} 13.0 (no split 16.6, {8, 4} 73).
 constexpr int64_t kPgSmallBytes = (int64_t)80 << 20;
 // a launch has less than 2^32 threads in x; the prep takes 256 a row
@@ -1942,7 +1944,10 @@ static int launch_skv(const void *hidden, int ht, int64_t rows, int64_t K, const
     // fewer columns leave CUs idle at any width; the stages of a tile are then
     // a chain of load latencies, shorter with half the loads per stage (bf16,
     // us: V 16379 K 2752 40.0 at 256 columns, 32.3 at 128, 34.0 at 64, 58 at
-    // 32; V 8000 K 4096 57.0, 48.7, 49.0, 51.7; V 3000 K 4096 46.3, 41.6)
+    // 32; V 8000 K 4096 57.0, 48.7, 49.0, 51.7; V 3000 K 4096 46.3, 41.6). fp32
+    // is bound by its MFMAs above 16 rows: V 8000 K 4096, 16 rows 92.7 at 256,
+    // 89.0 at 128, 88.8 at 64, 64 rows 261.9, 261.1, 261.7; V 16000 K 2048, 16
+    // rows 51.8, 49.8, 51.9, 32 rows 76.3, 77.9, 81.3
     tw = kSkvBN / 2;
   }
   const int64_t ntiles = (V + tw - 1) / tw;
@@ -2041,7 +2046,7 @@ static int launch_vgen(const void *hidden, int ht, int64_t rows, int64_t K, cons
 }
 
 // Route: the persistent streaming kernel (one dtype for hidden and W:
-// BF16, F16 or F32; any bias; 128-byte stages of whole ring rounds; 16-byte
+// BF16, F16 or F32; any bias; whole 128-byte stages, see skv_usable; 16-byte
 // aligned), else the column-group streaming kernel (same dtype for hidden
 // and W, 16-byte rows and pointers), else the generic kernel.
 static int verify_route(const void *hidden, int ht, int64_t rows, int64_t K, const void *w,
