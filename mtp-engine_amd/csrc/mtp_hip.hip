@@ -1352,11 +1352,12 @@ void plan_dec_16bit(DecPlan &p, int64_t units, int64_t keys, int64_t D) {
   constexpr double kCuRate = 57.7e3, kChipRate = 6.85e6;  // bytes per us
   constexpr double kMerge = 0.96, kMergeChunk = 0.066;
   const int maxw = dec_max_waves(MTP_BF16);
+  const int64_t cus = device_cus();
   const int64_t blocks = (keys + kAttnBlock - 1) / kAttnBlock;
   const int64_t step = 64 / (D / 8) * kDecLoads;  // keys of a wave's step
   double best = 0;
   for (int nw = maxw; nw >= 4; nw /= 2) {
-    const int64_t slots = (int64_t)device_cus() * maxw / nw;
+    const int64_t slots = cus * maxw / nw;
     for (int64_t want : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
       int64_t cb = dec_chunk_blocks((blocks + want - 1) / want, blocks);
       int64_t nc = (blocks + cb - 1) / cb;
@@ -1366,7 +1367,7 @@ void plan_dec_16bit(DecPlan &p, int64_t units, int64_t keys, int64_t D) {
       }
       const int64_t ck = std::min(keys, cb * kAttnBlock), groups = units * nc;
       const double bytes = (double)(ck * D * 4);  // K and V of a workgroup
-      const int64_t percu = std::min<int64_t>(maxw / nw, (groups + device_cus() - 1) / device_cus());
+      const int64_t percu = std::min<int64_t>(maxw / nw, (groups + cus - 1) / cus);
       const double chain = kStep * (double)((ck + step * nw - 1) / (step * nw));
       const double cu = (double)percu * bytes / kCuRate;
       const double chip = (double)std::min(groups, slots) * bytes / kChipRate;
@@ -1383,6 +1384,36 @@ void plan_dec_16bit(DecPlan &p, int64_t units, int64_t keys, int64_t D) {
       if (want >= blocks || units > kCounterSlots) break;
     }
   }
+}
+
+// The plan depends on the sizes, the CU count and the tuning keys alone; a
+// thread keeps its last few: the search is 0.8 us of host time, and a call
+// asks for its plan twice (workspace size and launch).
+void make_plan_dec_16bit(DecPlan &p, int64_t units, int64_t keys, int64_t D) {
+  struct Entry {
+    int64_t units = -1, keys = 0, D = 0;
+    int cus = 0, waves = 0, nchunks = 0, chunk_blocks = 0;
+    unsigned epoch = 0;
+  };
+  constexpr int kEntries = 16;
+  static thread_local Entry cache[kEntries];
+  const unsigned epoch = tune_epoch();
+  const int cus = device_cus();
+  Entry &e = cache[(unsigned)(units * 31 + keys * 7 + D / 64) % kEntries];
+  if (e.units != units || e.keys != keys || e.D != D || e.cus != cus || e.epoch != epoch) {
+    plan_dec_16bit(p, units, keys, D);
+    e.units = units;
+    e.keys = keys;
+    e.D = D;
+    e.cus = cus;
+    e.waves = p.waves;
+    e.nchunks = p.nchunks;
+    e.chunk_blocks = p.chunk_blocks;
+    e.epoch = epoch;
+  }
+  p.waves = e.waves;
+  p.nchunks = e.nchunks;
+  p.chunk_blocks = e.chunk_blocks;
 }
 
 // What a merge of chunks costs (partials through the device coherence point,
@@ -1440,7 +1471,7 @@ DecPlan make_dec_plan(int ct, int64_t B, int64_t NQ, int64_t H, int64_t D, int64
   const int64_t blocks = (Lc + Lt + kAttnBlock - 1) / kAttnBlock;
   if (blocks == 0) return p;  // no key: rows of 0 / 0
   if ((ct == MTP_BF16 || ct == MTP_F16) && D != 256 && NQ == 1 && !kv_fp8)
-    plan_dec_16bit(p, units, Lc + Lt, D);
+    make_plan_dec_16bit(p, units, Lc + Lt, D);
   else
     plan_dec_other(p, units, blocks, maxw);
   if (p.nchunks > 1) {
