@@ -1,5 +1,7 @@
 """Launch plans seen from the host (CPU): what the workspace queries ask for.
 Without a device the plans are made for 256 CUs."""
+import threading
+
 import pytest
 
 from mtp_hip import _lib as L
@@ -20,6 +22,35 @@ def test_decode_attention_has_at_most_64_chunks(lib, dtype, D, keys, chunk):
         n = lib.mtp_attention_workspace_bytes(dtype, 1, 1, 3, D, 0, keys)
     most = L.MTP_COUNTER_BYTES + 3 * 64 * (D + 2) * 4
     assert n <= -(-most // 256) * 256
+
+
+def test_kept_decode_plans_are_of_their_sizes_and_keys(lib):
+    """The plans a thread keeps: more sizes than it holds, asked for in both
+    orders, against a thread that has none; a tuning key set in between. At more
+    than 128 heads the MFMA kernel's plan has one chunk and no workspace, so the
+    query shows the decode kernel's chunks."""
+    sizes = [(H, D, keys) for D in (64, 128) for H in (160, 257, 288, 384)
+             for keys in (65, 511, 700, 1024, 1500, 2272, 4096)]
+
+    def ask(size):
+        H, D, keys = size
+        return lib.mtp_attention_workspace_bytes(L.BF16, 1, 1, H, D, 0, keys)
+
+    def ask_anew(size):
+        got = []
+        t = threading.Thread(target=lambda: got.append(ask(size)))
+        t.start()
+        t.join()
+        return got[0]
+
+    fresh = {size: ask_anew(size) for size in sizes}
+    assert len(set(fresh.values())) > 8  # plans of several chunk counts
+    assert [ask(s) for s in sizes] == [fresh[s] for s in sizes]
+    assert [ask(s) for s in sizes[::-1]] == [fresh[s] for s in sizes[::-1]]
+    last = sizes[-1]
+    with L.tuning(attn_chunk_blocks=1):
+        assert ask(last) == ask_anew(last) != fresh[last]
+    assert ask(last) == fresh[last]
 
 
 @pytest.mark.parametrize("w", [L.BF16, L.FP8E4M3])
